@@ -6,6 +6,7 @@
 
 #include <atomic>
 #include <string>
+#include <vector>
 
 #include "fmath.h"
 #include "vdsl.h"
@@ -39,6 +40,8 @@ struct vdsl_queue_s {
   vdsl_device dev;
   hipStream_t stream;
   bool capturing;
+  void* scratch = nullptr;            // queue_scratch(): kept from the first op that asks for it
+  std::vector<void*> graph_scratch;   // asked for by the ops recorded since vdsl_graph_begin
 };
 
 struct vdsl_graph_s {
@@ -46,6 +49,7 @@ struct vdsl_graph_s {
   vdsl_device dev;
   hipGraph_t graph;
   hipGraphExec_t exec;
+  std::vector<void*> scratch;  // of its ops; freed with it
 };
 
 struct vdsl_event_s {
@@ -74,6 +78,14 @@ int enter_queue(vdsl_queue q);
 int check_buffer(vdsl_queue q, vdsl_buffer b, size_t bytes, const char* name, bool writable);
 
 size_t dtype_size(int dtype);
+
+// Device memory for one op's partial results on queue q, valid until the queue's next op: the
+// queue's own kQueueScratchBytes, allocated when first asked for, or, while q records a graph, a
+// piece of its own that the graph then owns (so graphs replayed on any queues share nothing).
+// *out is null, with VDSL_OK, when `bytes` is more than that or cannot be had: the op then takes
+// the path that needs none.
+constexpr size_t kQueueScratchBytes = size_t{1} << 20;
+int queue_scratch(vdsl_queue q, size_t bytes, void** out);
 
 // Per-device set-up of the allocation-free int8 GEMM (gemm_w8a8.hip); called by vdsl_device_open
 // with the device current.

@@ -20,6 +20,8 @@
 // rows and needs no LDS and no barrier.  Widths that are not one of the register-resident
 // shapes use a 3-pass streaming kernel (max/sum, exp-sum, write) with the same arithmetic.
 
+#include <type_traits>
+
 #include "common.h"
 
 namespace vdsl {
@@ -300,34 +302,207 @@ __global__ __launch_bounds__(256) void row_softmax_generic(const void* __restric
   for (int64_t c = lane; c < cols; c += 64) E::store1(sm, base + c, expf(E::load1(x, base + c) - m) / esf);
 }
 
-// Column reductions: a block owns 64 columns; 4 row groups accumulate in f64 and are combined in
-// a fixed order, so results do not depend on scheduling.
-template <int DT>
-__global__ __launch_bounds__(256) void col_reduce_kernel(const void* __restrict__ x, float* __restrict__ col_sum,
-                                                         float* __restrict__ col_max, int64_t rows, int64_t cols) {
+// Column reductions.  A block owns a strip of L * VEC columns (L a power of two, VEC elements per
+// load) and a range of rows: its 1024 lanes are L column lanes x 1024 / L row lanes, each adding
+// its rows in f64 in row order; the row lanes then meet in a fixed order (butterflies in the wave,
+// the 16 waves in LDS), so results do not depend on scheduling.  With one range the block stores
+// the result; with several it stores f64 sums and f32 maxima to scratch memory and
+// col_finish_kernel adds the ranges in order.
+constexpr int kColThreads = 1024, kColBatch = 8;
+
+// VEC consecutive elements of a row from one load (16 bytes, a bf16 pair or one element).
+template <int DT, int VEC>
+struct ColLoad {
   using E = Elem<DT>;
-  __shared__ double ssum[4][64];
-  __shared__ float smax[4][64];
-  const int c_local = threadIdx.x & 63;
-  const int g = threadIdx.x >> 6;
-  const int64_t c = static_cast<int64_t>(blockIdx.x) * 64 + c_local;
+  static constexpr int kBytes = VEC * (DT == VDSL_F32 ? 4 : 2);
+  using Raw = std::conditional_t<kBytes == 16, u32x4, std::conditional_t<kBytes == 4, uint32_t, uint16_t>>;
+  __device__ static __forceinline__ void unpack(const Raw& r, float (&o)[VEC]) {
+    if constexpr (kBytes == 16) {
+      E::unpack(make_uint4(r[0], r[1], r[2], r[3]), o);
+    } else if constexpr (DT == VDSL_F32) {
+      o[0] = __uint_as_float(r);
+    } else if constexpr (VEC == 2) {
+      o[0] = __uint_as_float(r << 16);
+      o[1] = __uint_as_float(r & 0xFFFF0000u);
+    } else {
+      o[0] = bf16_to_f32(r);
+    }
+  }
+};
+
+template <int DT, int VEC>
+__global__ __launch_bounds__(kColThreads) void col_reduce_kernel(const void* __restrict__ x, float* __restrict__ col_sum,
+                                                                 float* __restrict__ col_max, double* __restrict__ part_sum,
+                                                                 float* __restrict__ part_max, int64_t all_rows, int64_t per_range,
+                                                                 int64_t cols, int lg_lanes) {
+  using LD = ColLoad<DT, VEC>;
+  using Raw = typename LD::Raw;
+  extern __shared__ __align__(16) char col_smem[];  // [16][L * VEC] f64 sums, then as many f32 maxima
+  const int L = 1 << lg_lanes, width = VEC << lg_lanes, R = kColThreads >> lg_lanes;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t strip = blockIdx.x, first = static_cast<int64_t>(blockIdx.y) * per_range;
+  const int64_t rows = all_rows - first < per_range ? all_rows - first : per_range;  // of this range
+  const int cl = threadIdx.x & (L - 1);
+  const int64_t rl = threadIdx.x >> lg_lanes;
+  const int64_t c = strip * width + cl * VEC;
+  const int64_t pitch = cols / VEC;  // cols % VEC == 0
+  const Raw* src = reinterpret_cast<const Raw*>(x) + first * pitch + c / VEC;
+  double s[VEC];
+  float m[VEC];
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) s[e] = 0.0, m[e] = -INFINITY;
+  if (c < cols) {
+    int64_t r = rl;
+    for (; r + static_cast<int64_t>(kColBatch - 1) * R < rows; r += static_cast<int64_t>(kColBatch) * R) {
+      Raw v[kColBatch];
+#pragma unroll
+      for (int u = 0; u < kColBatch; ++u) v[u] = src[(r + static_cast<int64_t>(u) * R) * pitch];
+#pragma unroll
+      for (int u = 0; u < kColBatch; ++u) {
+        float f[VEC];
+        LD::unpack(v[u], f);
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+          s[e] += static_cast<double>(f[e]);
+          m[e] = fmaxf(m[e], f[e]);
+        }
+      }
+    }
+    if (r < rows) {  // the last, partial batch: rows past the end read the last row and add nothing
+      Raw v[kColBatch];
+#pragma unroll
+      for (int u = 0; u < kColBatch; ++u) {
+        const int64_t ru = r + static_cast<int64_t>(u) * R;
+        v[u] = src[(ru < rows ? ru : rows - 1) * pitch];
+      }
+#pragma unroll
+      for (int u = 0; u < kColBatch; ++u) {
+        const bool in = r + static_cast<int64_t>(u) * R < rows;
+        float f[VEC];
+        LD::unpack(v[u], f);
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+          s[e] += static_cast<double>(in ? f[e] : 0.0f);
+          m[e] = fmaxf(m[e], in ? f[e] : -INFINITY);
+        }
+      }
+    }
+  }
+  for (int k = 32; k >= L; k >>= 1) {
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      s[e] += __shfl_xor(s[e], k, 64);
+      m[e] = fmaxf(m[e], __shfl_xor(m[e], k, 64));
+    }
+  }
+  double* const ssum = reinterpret_cast<double*>(col_smem);
+  float* const smax = reinterpret_cast<float*>(ssum + (kColThreads / 64) * width);
+  if (lane < L) {
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      ssum[wave * width + cl * VEC + e] = s[e];
+      smax[wave * width + cl * VEC + e] = m[e];
+    }
+  }
+  __syncthreads();
+  for (int k = threadIdx.x; k < width; k += kColThreads) {
+    const int64_t col = strip * width + k;
+    if (col >= cols) break;
+    double t = ssum[k];
+    float mm = smax[k];
+#pragma unroll
+    for (int w = 1; w < kColThreads / 64; ++w) {
+      t += ssum[w * width + k];
+      mm = fmaxf(mm, smax[w * width + k]);
+    }
+    if (part_sum) {
+      part_sum[blockIdx.y * cols + col] = t;
+      part_max[blockIdx.y * cols + col] = mm;
+    } else {
+      if (col_sum) col_sum[col] = static_cast<float>(t);
+      if (col_max) col_max[col] = mm;
+    }
+  }
+}
+
+// Adds the row ranges' partial results: 64 columns per block, its 16 waves taking every 16th range
+// of them and meeting in LDS, both in a fixed order.
+__global__ __launch_bounds__(kColThreads) void col_finish_kernel(const double* __restrict__ part_sum,
+                                                                 const float* __restrict__ part_max,
+                                                                 float* __restrict__ col_sum, float* __restrict__ col_max,
+                                                                 int64_t cols, int ranges) {
+  constexpr int W = kColThreads / 64;
+  __shared__ double ssum[W][64];
+  __shared__ float smax[W][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t c = static_cast<int64_t>(blockIdx.x) * 64 + lane;
   double s = 0.0;
   float m = -INFINITY;
-  if (c < cols)
-    for (int64_t r = g; r < rows; r += 4) {
-      const float v = E::load1(x, r * cols + c);
-      s += static_cast<double>(v);
-      m = fmaxf(m, v);
+  if (c < cols) {
+#pragma unroll 4
+    for (int k = wave; k < ranges; k += W) {
+      s += part_sum[k * cols + c];
+      m = fmaxf(m, part_max[k * cols + c]);
     }
-  ssum[g][c_local] = s;
-  smax[g][c_local] = m;
-  __syncthreads();
-  if (g == 0 && c < cols) {
-    const double t = ((ssum[0][c_local] + ssum[1][c_local]) + ssum[2][c_local]) + ssum[3][c_local];
-    const float mm = fmaxf(fmaxf(smax[0][c_local], smax[1][c_local]), fmaxf(smax[2][c_local], smax[3][c_local]));
-    if (col_sum) col_sum[c] = static_cast<float>(t);
-    if (col_max) col_max[c] = mm;
   }
+  ssum[wave][lane] = s;
+  smax[wave][lane] = m;
+  __syncthreads();
+  if (wave == 0 && c < cols) {
+#pragma unroll
+    for (int w = 1; w < W; ++w) {
+      s += ssum[w][lane];
+      m = fmaxf(m, smax[w][lane]);
+    }
+    if (col_sum) col_sum[c] = static_cast<float>(s);
+    if (col_max) col_max[c] = m;
+  }
+}
+
+// The strip's width (log2 of its column lanes) and the row ranges.  A CU misses its L1 at about one
+// 128-byte line per 4 cycles whatever part of the line is used, so strips of 256 bytes of a row are
+// read best, and row ranges make them cover the CUs: [16384][4096] f32 1627 us with one block of
+// 256 lanes per 64 columns, 70.3-78.5 us in one launch with 64- or 128-byte strips, 47.8 us (5616
+// GB/s) with 256-byte strips in 8 ranges (512 blocks; 256 blocks 51.1, 1024 49.1); bf16 27.2 us
+// with 256 blocks (512: 30.0); [16384][256] f32 8.5 us against 31 us in one launch.  For less the
+// second launch costs more than the strips' latency ([700][700] f32 6.8 us a call against 5.4; but
+// [16384][64] 7.2 against 21.7, hence the row count): one range, and strips narrowed to 16 bytes
+// while they do not cover the CUs and a row lane has more than half a batch of rows.
+template <int DT, int VEC>
+int launch_cols(vdsl_queue q, const void* x, float* cs, float* cm, int64_t rows, int64_t cols) {
+  constexpr int kBytes = ColLoad<DT, VEC>::kBytes;
+  const auto strips = [&](int l) { return (cols + (int64_t{VEC} << l) - 1) / (int64_t{VEC} << l); };
+  const int64_t bytes = rows * cols * (DT == VDSL_F32 ? 4 : 2);  // fits: checked by the caller
+  int lg = kBytes == 16 ? 4 : 6, ranges = 1;
+  int64_t per_range = rows;
+  double* part = nullptr;
+  if (bytes >= (int64_t{4} << 20) || (bytes >= (int64_t{1} << 20) && rows >= 4096)) {
+    const int64_t by_blocks = (DT == VDSL_F32 && bytes >= (int64_t{128} << 20) ? 512 : 256) / strips(lg);
+    const int64_t by_rows = rows / (kColBatch / 2 * (kColThreads >> lg));
+    const int64_t want = by_blocks < by_rows ? by_blocks : by_rows;
+    if (want > 1) {
+      per_range = (rows + want - 1) / want;
+      ranges = static_cast<int>((rows + per_range - 1) / per_range);
+      void* scratch = nullptr;
+      VDSL_TRY(queue_scratch(q, nbytes(ranges, cols, 12), &scratch));
+      part = static_cast<double*>(scratch);
+    }
+  }
+  if (!part) {
+    ranges = 1, per_range = rows, lg = 6;
+    while (lg > 0 && (kBytes << (lg - 1)) >= 16 && strips(lg) < 256 && rows > (kColBatch / 2) * (kColThreads >> lg)) --lg;
+  }
+  const int64_t blocks = strips(lg);
+  if (blocks > 0x7fffffff) return fail(VDSL_ERR_UNSUPPORTED, "too many columns");
+  float* pmax = part ? reinterpret_cast<float*>(part + static_cast<int64_t>(ranges) * cols) : nullptr;
+  const unsigned lds = static_cast<unsigned>((kColThreads / 64) * (VEC << lg) * 12);
+  hipLaunchKernelGGL((col_reduce_kernel<DT, VEC>), dim3(static_cast<unsigned>(blocks), static_cast<unsigned>(ranges)),
+                     dim3(kColThreads), lds, q->stream, x, cs, cm, part, pmax, rows, per_range, cols, lg);
+  VDSL_TRY(check_launch("col_reduce_kernel"));
+  if (!part) return VDSL_OK;
+  hipLaunchKernelGGL(col_finish_kernel, dim3(static_cast<unsigned>((cols + 63) / 64)), dim3(kColThreads), 0, q->stream, part, pmax,
+                     cs, cm, cols, ranges);
+  return check_launch("col_finish_kernel");
 }
 
 template <int DT>
@@ -405,12 +580,14 @@ extern "C" int vdsl_op_col_reduce(vdsl_queue q, int64_t rows, int64_t cols, int3
   if (col_sum) VDSL_TRY(check_buffer(q, col_sum, nbytes(cols, 4), "col_sum", true));
   if (col_max) VDSL_TRY(check_buffer(q, col_max, nbytes(cols, 4), "col_max", true));
   if (cols == 0) return VDSL_OK;
-  const int64_t blocks = (cols + 63) / 64;
   float* cs = col_sum ? static_cast<float*>(col_sum->ptr) : nullptr;
   float* cm = col_max ? static_cast<float*>(col_max->ptr) : nullptr;
-  if (dtype == VDSL_F32)
-    hipLaunchKernelGGL((col_reduce_kernel<VDSL_F32>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, q->stream, x->ptr, cs, cm, rows, cols);
-  else
-    hipLaunchKernelGGL((col_reduce_kernel<VDSL_BF16>), dim3(static_cast<unsigned>(blocks)), dim3(256), 0, q->stream, x->ptr, cs, cm, rows, cols);
-  return check_launch("col_reduce_kernel");
+  // 16-byte loads need rows of whole 16-byte units (hipMalloc bases are aligned).
+  if (dtype == VDSL_F32) {
+    if (cols % 4 == 0) return launch_cols<VDSL_F32, 4>(q, x->ptr, cs, cm, rows, cols);
+    return launch_cols<VDSL_F32, 1>(q, x->ptr, cs, cm, rows, cols);
+  }
+  if (cols % 8 == 0) return launch_cols<VDSL_BF16, 8>(q, x->ptr, cs, cm, rows, cols);
+  if (cols % 2 == 0) return launch_cols<VDSL_BF16, 2>(q, x->ptr, cs, cm, rows, cols);
+  return launch_cols<VDSL_BF16, 1>(q, x->ptr, cs, cm, rows, cols);
 }

@@ -109,6 +109,32 @@ int check_buffer(vdsl_queue q, vdsl_buffer b, size_t bytes, const char* name, bo
   return VDSL_OK;
 }
 
+int queue_scratch(vdsl_queue q, size_t bytes, void** out) {
+  *out = nullptr;
+  if (!bytes || bytes > kQueueScratchBytes) return VDSL_OK;
+  if (!q->capturing) {
+    if (!q->scratch && hipMalloc(&q->scratch, kQueueScratchBytes) != hipSuccess) {
+      (void)hipGetLastError();
+      q->scratch = nullptr;
+    }
+    *out = q->scratch;
+    return VDSL_OK;
+  }
+  // An allocation does not touch the recording; the thread's capture mode has to allow it.
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  VDSL_TRY(check_hip(hipThreadExchangeStreamCaptureMode(&mode), "hipThreadExchangeStreamCaptureMode"));
+  void* p = nullptr;
+  const hipError_t e = hipMalloc(&p, bytes);
+  VDSL_TRY(check_hip(hipThreadExchangeStreamCaptureMode(&mode), "hipThreadExchangeStreamCaptureMode"));
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    return VDSL_OK;
+  }
+  q->graph_scratch.push_back(p);
+  *out = p;
+  return VDSL_OK;
+}
+
 size_t dtype_size(int dtype) {
   switch (dtype) {
     case VDSL_F32: return 4;
@@ -348,6 +374,7 @@ int vdsl_queue_destroy(vdsl_queue q) {
   (void)hipSetDevice(q->dev->ordinal);
   int st = check_hip(hipStreamSynchronize(q->stream), "hipStreamSynchronize");
   (void)hipStreamDestroy(q->stream);
+  if (q->scratch) (void)hipFree(q->scratch);
   reg_del(q);
   q->dev->live.fetch_sub(1);
   q->magic = 0;
@@ -377,16 +404,27 @@ int vdsl_graph_end(vdsl_queue q, vdsl_graph* out) {
   VDSL_TRY(enter_queue(q));
   if (!q->capturing) return fail(VDSL_ERR_CAPTURE, "graph_end without graph_begin");
   q->capturing = false;
+  std::vector<void*> scratch;
+  scratch.swap(q->graph_scratch);
+  auto drop = [&]() {
+    for (void* p : scratch) (void)hipFree(p);
+  };
   hipGraph_t g = nullptr;
-  VDSL_TRY(check_hip(hipStreamEndCapture(q->stream, &g), "hipStreamEndCapture"));
+  int st = check_hip(hipStreamEndCapture(q->stream, &g), "hipStreamEndCapture");
+  if (st != VDSL_OK) {
+    drop();
+    return st;
+  }
   if (!out) {
     (void)hipGraphDestroy(g);
+    drop();
     return fail(VDSL_ERR_INVALID_ARG, "out is null (recording discarded)");
   }
   hipGraphExec_t exec = nullptr;
-  int st = check_hip(hipGraphInstantiate(&exec, g, nullptr, nullptr, 0), "hipGraphInstantiate");
+  st = check_hip(hipGraphInstantiate(&exec, g, nullptr, nullptr, 0), "hipGraphInstantiate");
   if (st != VDSL_OK) {
     (void)hipGraphDestroy(g);
+    drop();
     return st;
   }
   auto* gr = new vdsl_graph_s();
@@ -394,6 +432,7 @@ int vdsl_graph_end(vdsl_queue q, vdsl_graph* out) {
   gr->dev = q->dev;
   gr->graph = g;
   gr->exec = exec;
+  gr->scratch = std::move(scratch);
   q->dev->live.fetch_add(1);
   reg_add(gr);
   *out = gr;
@@ -413,6 +452,7 @@ int vdsl_graph_destroy(vdsl_graph g) {
   (void)hipSetDevice(g->dev->ordinal);
   (void)hipGraphExecDestroy(g->exec);
   (void)hipGraphDestroy(g->graph);
+  for (void* p : g->scratch) (void)hipFree(p);
   reg_del(g);
   g->dev->live.fetch_sub(1);
   g->magic = 0;
