@@ -5,7 +5,7 @@
 //   row_max = max_j x[j] (exact);
 //   softmax[j] = e[j] / s,  e[j] = exp(x[j] - row_max) in f32,  s = f64 sum of e rounded to f32.
 // (The register-resident kernels evaluate exp with the branch-free exp_fast of fmath.h, in its
-// form for arguments <= 0, within a few ulp of the library expf that the generic kernel and the
+// form for arguments <= 0, within a few ulp of the library expf that the streaming kernel and the
 // oracle use.)
 // The register-resident kernels multiply by 1/s instead of dividing (within one ulp of e/s) and
 // form their sums as f32 partials of 4 or 8 elements added into f64 accumulators (f32 rows) or,
@@ -17,8 +17,9 @@
 // and softmax written once (the HBM roofline's minimum traffic).  Lane l holds the 16-byte
 // vectors v*64 + l, v < NV, so every load/store instruction of a wave covers 1 KiB contiguous.
 // Reductions stay inside the wave (xor butterflies), so a 256-thread block is 4 independent
-// rows and needs no LDS and no barrier.  Widths that are not one of the register-resident
-// shapes use a 3-pass streaming kernel (max/sum, exp-sum, write) with the same arithmetic.
+// rows and needs no LDS and no barrier.  Other widths are held in registers too, masked at their
+// ends (row_softmax_any); only rows wider than 8192 vectors use a 3-pass streaming kernel
+// (max/sum, exp-sum, write).
 
 #include <type_traits>
 
@@ -272,7 +273,166 @@ __global__ __launch_bounds__(64 * WPR) void row_softmax_split(const void* __rest
   }
 }
 
-// Any width: three streaming passes over the row with the same arithmetic.
+// exp of n[0 .. PV) <= 0, the steps of exp_fast.  Where some lane of the wave has an n below -87, whose
+// exp2 would be flushed or whose exponent may be infinite, the wave takes the form that keeps
+// subnormal results: the power is formed 2^32 higher (t + 32 is exact there) and scaled back once.
+// NaN becomes 0 there: the caller gives a row with a NaN or an infinite maximum NaN.
+template <int PV>
+__device__ __forceinline__ void exp_nonpos_vec(float (&n)[PV]) {
+  float low = n[0];
+#pragma unroll
+  for (int e = 1; e < PV; ++e) low = fminf(low, n[e]);
+  if (__any(low < -87.0f)) {
+#pragma unroll
+    for (int e = 0; e < PV; ++e) {
+      const float c = fmaxf(n[e], -200.0f);
+      const float t = c * 1.4426950408889634f;
+      float r = __builtin_fmaf(c, 1.4426950408889634f, -t);
+      r = __builtin_fmaf(c, 1.92596299e-08f, r);  // log2(e) - fl(log2(e))
+      const bool up = t < -100.0f;
+      const float x = __builtin_amdgcn_exp2f(up ? t + 32.0f : t);
+      n[e] = __builtin_ldexpf(__builtin_fmaf(x, r * 0.6931471805599453f, x), up ? -32 : 0);
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < PV; ++e) {
+      const float t = n[e] * 1.4426950408889634f;
+      float r = __builtin_fmaf(n[e], 1.4426950408889634f, -t);
+      r = __builtin_fmaf(n[e], 1.92596299e-08f, r);
+      const float x = __builtin_amdgcn_exp2f(t);
+      n[e] = __builtin_fmaf(x, r * 0.6931471805599453f, x);
+    }
+  }
+}
+
+// e / s from i = 1 / s (correctly rounded): the rounded product corrected once by its exact
+// residual (Markstein), which rounds normal results correctly in 3 operations.
+__device__ __forceinline__ float quotient(float e, float s, float i) {
+  const float q = e * i;
+  return __builtin_fmaf(__builtin_fmaf(-q, s, e), i, q);
+}
+
+// Any width up to NV 16-byte vectors per lane: the row is read once, in the aligned vectors that
+// cover it (a row of an odd width starts anywhere in its first vector), and held in registers.
+// Elements of the first and last vector that belong to the neighbouring rows are read with it,
+// replaced by -inf and never stored; only the tensor's very last vector is read by elements.  BLOCK:
+// a block per row, its waves meeting in LDS; else groups of 1 << lg_lanes <= 64 lanes take a row
+// each and reduce by butterflies.  Sums are f64 sums of every element, as in the streaming kernel.
+// Bound by HBM for f32 and by VALU work (the f64 sums and the exponential) for bf16.  [3000][5003]
+// f32: 99.4 us with the streaming kernel (three passes of 4-byte loads, one wave per row), 23.3 us
+// (5.16 TB/s) here; bf16 76 -> 20 us; [16384][1000] f32 58.8 -> 26 us.
+template <int DT, int NV, bool BLOCK>
+__global__ __launch_bounds__(BLOCK ? 1024 : 256) void row_softmax_any(const void* __restrict__ x, float* __restrict__ row_sum,
+                                                                      float* __restrict__ row_max, void* __restrict__ sm,
+                                                                      int64_t rows, int64_t cols, int lg_lanes) {
+  using E = Elem<DT>;
+  constexpr int PV = E::kPerVec;
+  __shared__ double part_sum[BLOCK ? 16 : 1];
+  __shared__ float part_max[BLOCK ? 16 : 1];
+  const int lanes = BLOCK ? static_cast<int>(blockDim.x) : 1 << lg_lanes;  // per row
+  const int at = BLOCK ? static_cast<int>(threadIdx.x) : static_cast<int>(threadIdx.x) & (lanes - 1);
+  const int64_t row = BLOCK ? static_cast<int64_t>(blockIdx.x)
+                            : static_cast<int64_t>(blockIdx.x) * (256 >> lg_lanes) + (threadIdx.x >> lg_lanes);
+  const bool live = row < rows;  // groups past the last row take part in the wave's butterflies
+  const int64_t begin = row * cols, end = begin + cols, total = rows * cols;
+  const int64_t first = begin / PV;
+  const int waves = lanes >> 6, wave = threadIdx.x >> 6;
+
+  float v[NV][PV];
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    const int64_t i = first + at + static_cast<int64_t>(k) * lanes, e0 = i * PV;
+    if (live && e0 < end) {
+      if (e0 + PV <= total) {
+        const u32x4 r = __builtin_nontemporal_load(static_cast<const u32x4*>(x) + i);
+        E::unpack(make_uint4(r[0], r[1], r[2], r[3]), v[k]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < PV; ++e) v[k][e] = e0 + e < total ? E::load1(x, e0 + e) : 0.0f;
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < PV; ++e) v[k][e] = 0.0f;
+    }
+  }
+  double s = 0.0;
+  float m = -INFINITY;
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    const int64_t e0 = (first + at + static_cast<int64_t>(k) * lanes) * PV;
+    if (e0 >= begin && e0 + PV <= end) {
+#pragma unroll
+      for (int e = 0; e < PV; ++e) {
+        s += static_cast<double>(v[k][e]);
+        m = fmaxf(m, v[k][e]);
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < PV; ++e) {
+        const bool in = e0 + e >= begin && e0 + e < end;
+        s += static_cast<double>(in ? v[k][e] : 0.0f);
+        v[k][e] = in ? v[k][e] : -INFINITY;
+        m = fmaxf(m, v[k][e]);
+      }
+    }
+  }
+  // The row's f64 sum of one value per lane, on every lane; the same order on each.
+  const auto row_total = [&](double t) -> double {
+    for (int d = (BLOCK ? 64 : lanes) >> 1; d >= 1; d >>= 1) t += __shfl_xor(t, d, 64);
+    if constexpr (BLOCK) {
+      if ((threadIdx.x & 63) == 0) part_sum[wave] = t;
+      __syncthreads();
+      t = 0.0;
+      for (int w = 0; w < waves; ++w) t += part_sum[w];
+    }
+    return t;
+  };
+  for (int d = (BLOCK ? 64 : lanes) >> 1; d >= 1; d >>= 1) m = fmaxf(m, __shfl_xor(m, d, 64));
+  if constexpr (BLOCK) {
+    if ((threadIdx.x & 63) == 0) part_max[wave] = m;
+  }
+  s = row_total(s);
+  if constexpr (BLOCK) {
+    for (int w = 0; w < waves; ++w) m = fmaxf(m, part_max[w]);
+  }
+  if (live && at == 0) {
+    if (row_sum) row_sum[row] = static_cast<float>(s);
+    if (row_max) row_max[row] = m;
+  }
+  if (!sm) return;
+  double es = 0.0;
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+#pragma unroll
+    for (int e = 0; e < PV; ++e) v[k][e] = v[k][e] - m;
+    exp_nonpos_vec<PV>(v[k]);
+#pragma unroll
+    for (int e = 0; e < PV; ++e) es += static_cast<double>(v[k][e]);
+  }
+  if constexpr (BLOCK) __syncthreads();  // every wave has read part_sum
+  // A NaN element (its sum is NaN), +inf or a row of -inf: every quotient is NaN.
+  const bool nan_row = __builtin_isnan(s) || __builtin_isinf(m);
+  es = row_total(es);
+  const float sum = nan_row ? __builtin_nanf("") : static_cast<float>(es), inv = 1.0f / sum;
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    const int64_t i = first + at + static_cast<int64_t>(k) * lanes, e0 = i * PV;
+    if (!live || e0 >= end) continue;
+#pragma unroll
+    for (int e = 0; e < PV; ++e) v[k][e] = quotient(v[k][e], sum, inv);
+    if (e0 >= begin && e0 + PV <= end) {
+      const uint4 w = E::pack(v[k]);
+      const u32x4 wv = {w.x, w.y, w.z, w.w};
+      __builtin_nontemporal_store(wv, static_cast<u32x4*>(sm) + i);
+    } else {
+#pragma unroll
+      for (int e = 0; e < PV; ++e)
+        if (e0 + e >= begin && e0 + e < end) E::store1(sm, e0 + e, v[k][e]);
+    }
+  }
+}
+
+// Rows wider than row_softmax_any holds: three streaming passes with the same arithmetic.
 template <int DT>
 __global__ __launch_bounds__(256) void row_softmax_generic(const void* __restrict__ x, float* __restrict__ row_sum,
                                                            float* __restrict__ row_max, void* __restrict__ sm,
@@ -531,15 +691,63 @@ int launch_rows(const void* x, float* rs, float* rm, void* sm, int64_t rows, int
   const dim3 grid(static_cast<unsigned>(blocks)), block(256);
   switch (cols) {
 #define VDSL_ROW_CASE(NV) \
-  case 64 * NV * PV: hipLaunchKernelGGL((row_softmax_resident<DT, NV>), grid, block, 0, st, x, rs, rm, sm, rows); break;
+  case 64 * NV * PV: \
+    hipLaunchKernelGGL((row_softmax_resident<DT, NV>), grid, block, 0, st, x, rs, rm, sm, rows); \
+    return check_launch("row_softmax");
     VDSL_ROW_CASE(1)
     VDSL_ROW_CASE(2)
     VDSL_ROW_CASE(4)
 #undef VDSL_ROW_CASE
-    default:
-      hipLaunchKernelGGL((row_softmax_generic<DT>), grid, block, 0, st, x, rs, rm, sm, rows, cols);
+    default: break;
   }
-  return check_launch("row_softmax");
+  // Other widths: the vectors that cover a row (one more than its width where rows start anywhere).
+  const int64_t nvec = (cols + PV - 1) / PV + (cols % PV ? 1 : 0);
+  constexpr int64_t kBlockMax = 1024 * 8;
+  if (nvec > kBlockMax || rows > 0x7fffffff) {
+    hipLaunchKernelGGL((row_softmax_generic<DT>), grid, block, 0, st, x, rs, rm, sm, rows, cols);
+    return check_launch("row_softmax");
+  }
+  // Waves per row: the fewest whose lanes hold the row in kMost vectors each.  More vectors per lane
+  // mean fewer reductions and barriers per element, until their registers leave too few waves; wave
+  // counts that are no multiple of 4 load a CU's SIMDs unevenly (9 waves of 94 registers: one block
+  // per CU instead of two, [4000][16383] f32 152 us against 100).  f32 [3000][5003]: 4 waves of 5
+  // vectors 24.0 us, 3 of 8 25.5, 5 of 4 25.7, 10 of 2 31; bf16 [8000][7000]: 4 of 4 55 us, 7 of 2 60,
+  // 2 of 8 73; bf16 [4000][12000]: 8 of 3 47 us, 6 of 4 65, 3 of 8 65.
+  constexpr int kWaves[] = {1, 2, 4, 8, 12, 16};
+  constexpr int kMostF32[] = {4, 5, 5, 6, 6, 8}, kMostBf16[] = {5, 5, 4, 3, 3, 8};
+  const int* most = DT == VDSL_F32 ? kMostF32 : kMostBf16;
+  int w = 0;
+  while (nvec > int64_t{64} * kWaves[w] * most[w]) ++w;  // ends: nvec <= kBlockMax
+  if (w == 0) {
+    int lg = 6;
+    while (lg > 0 && nvec <= (int64_t{1} << (lg - 1))) --lg;
+    const dim3 g(static_cast<unsigned>((rows + (256 >> lg) - 1) / (256 >> lg)));
+    switch ((nvec + 63) / 64) {
+#define VDSL_ANY_CASE(NV) \
+  case NV: hipLaunchKernelGGL((row_softmax_any<DT, NV, false>), g, block, 0, st, x, rs, rm, sm, rows, cols, lg); break;
+      VDSL_ANY_CASE(1)
+      VDSL_ANY_CASE(2)
+      VDSL_ANY_CASE(3)
+      VDSL_ANY_CASE(4)
+      default: hipLaunchKernelGGL((row_softmax_any<DT, 5, false>), g, block, 0, st, x, rs, rm, sm, rows, cols, lg);
+#undef VDSL_ANY_CASE
+    }
+    return check_launch("row_softmax_any");
+  }
+  const dim3 g(static_cast<unsigned>(rows)), bl(static_cast<unsigned>(64 * kWaves[w]));
+  switch ((nvec + 64 * kWaves[w] - 1) / (64 * kWaves[w])) {
+#define VDSL_ANY_CASE(NV) \
+  case NV: hipLaunchKernelGGL((row_softmax_any<DT, NV, true>), g, bl, 0, st, x, rs, rm, sm, rows, cols, 6); break;
+    case 1:
+    VDSL_ANY_CASE(2)
+    VDSL_ANY_CASE(3)
+    VDSL_ANY_CASE(4)
+    VDSL_ANY_CASE(5)
+    VDSL_ANY_CASE(6)
+    default: hipLaunchKernelGGL((row_softmax_any<DT, 8, true>), g, bl, 0, st, x, rs, rm, sm, rows, cols, 6);
+#undef VDSL_ANY_CASE
+  }
+  return check_launch("row_softmax_any");
 }
 
 }  // namespace
