@@ -537,13 +537,14 @@ __global__ __launch_bounds__(kColThreads) void col_reduce_kernel(const void* __r
       }
 #pragma unroll
       for (int u = 0; u < kColBatch; ++u) {
-        const bool in = r + static_cast<int64_t>(u) * R < rows;
-        float f[VEC];
-        LD::unpack(v[u], f);
+        if (r + static_cast<int64_t>(u) * R < rows) {  // a branch: few rows skip the f64 work of the rest
+          float f[VEC];
+          LD::unpack(v[u], f);
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) {
-          s[e] += static_cast<double>(in ? f[e] : 0.0f);
-          m[e] = fmaxf(m[e], in ? f[e] : -INFINITY);
+          for (int e = 0; e < VEC; ++e) {
+            s[e] += static_cast<double>(f[e]);
+            m[e] = fmaxf(m[e], f[e]);
+          }
         }
       }
     }
@@ -627,7 +628,14 @@ __global__ __launch_bounds__(kColThreads) void col_finish_kernel(const double* _
 // with 256 blocks (512: 30.0); [16384][256] f32 8.5 us against 31 us in one launch.  For less the
 // second launch costs more than the strips' latency ([700][700] f32 6.8 us a call against 5.4; but
 // [16384][64] 7.2 against 21.7, hence the row count): one range, and strips narrowed to 16 bytes
-// while they do not cover the CUs and a row lane has more than half a batch of rows.
+// while they do not cover the CUs and a row lane has more than half a
+// batch of rows.  Those read an element or a bf16 pair per lane (col_small): with 16 bytes per lane
+// the f64 adds and butterflies of few blocks take longer than the loads ([100][16384] bf16 5.1 us a
+// call against 4.1).
+bool col_small(int64_t rows, int64_t bytes) {
+  return !(bytes >= (int64_t{4} << 20) || (bytes >= (int64_t{1} << 20) && rows >= 4096));
+}
+
 template <int DT, int VEC>
 int launch_cols(vdsl_queue q, const void* x, float* cs, float* cm, int64_t rows, int64_t cols) {
   constexpr int kBytes = ColLoad<DT, VEC>::kBytes;
@@ -636,7 +644,7 @@ int launch_cols(vdsl_queue q, const void* x, float* cs, float* cm, int64_t rows,
   int lg = kBytes == 16 ? 4 : 6, ranges = 1;
   int64_t per_range = rows;
   double* part = nullptr;
-  if (bytes >= (int64_t{4} << 20) || (bytes >= (int64_t{1} << 20) && rows >= 4096)) {
+  if (!col_small(rows, bytes)) {
     const int64_t by_blocks = (DT == VDSL_F32 && bytes >= (int64_t{128} << 20) ? 512 : 256) / strips(lg);
     const int64_t by_rows = rows / (kColBatch / 2 * (kColThreads >> lg));
     const int64_t want = by_blocks < by_rows ? by_blocks : by_rows;
@@ -791,11 +799,12 @@ extern "C" int vdsl_op_col_reduce(vdsl_queue q, int64_t rows, int64_t cols, int3
   float* cs = col_sum ? static_cast<float*>(col_sum->ptr) : nullptr;
   float* cm = col_max ? static_cast<float*>(col_max->ptr) : nullptr;
   // 16-byte loads need rows of whole 16-byte units (hipMalloc bases are aligned).
+  const bool wide = !col_small(rows, static_cast<int64_t>(nbytes(rows, cols, dtype_size(dtype))));
   if (dtype == VDSL_F32) {
-    if (cols % 4 == 0) return launch_cols<VDSL_F32, 4>(q, x->ptr, cs, cm, rows, cols);
+    if (wide && cols % 4 == 0) return launch_cols<VDSL_F32, 4>(q, x->ptr, cs, cm, rows, cols);
     return launch_cols<VDSL_F32, 1>(q, x->ptr, cs, cm, rows, cols);
   }
-  if (cols % 8 == 0) return launch_cols<VDSL_BF16, 8>(q, x->ptr, cs, cm, rows, cols);
+  if (wide && cols % 8 == 0) return launch_cols<VDSL_BF16, 8>(q, x->ptr, cs, cm, rows, cols);
   if (cols % 2 == 0) return launch_cols<VDSL_BF16, 2>(q, x->ptr, cs, cm, rows, cols);
   return launch_cols<VDSL_BF16, 1>(q, x->ptr, cs, cm, rows, cols);
 }
