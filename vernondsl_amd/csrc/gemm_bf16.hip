@@ -16,6 +16,7 @@
 #include "gemm_mfma.h"
 #include "gemm_bpk.h"
 #include "gemm_dma.h"
+#include "gemm_skinny.h"
 
 namespace vdsl {
 
@@ -473,6 +474,63 @@ __global__ __launch_bounds__(256) void gemm_bf16_nt_simple(const uint16_t* __res
   else static_cast<uint16_t*>(C)[idx] = f32_to_bf16(y);
 }
 
+// ---- products with a short side (gemm_skinny.h) -----------------------------------------------------
+// Epilogue kinds of one kernel: the forward ones (`epi` selects it), the two backward ones and
+// VDSL_EPI_GELU_DERIV, as bf16_epilogue's template arguments.
+enum { kSkinnyForward = 0, kSkinnyGeluBwd = 1, kSkinnyMul = 2, kSkinnyDeriv = 3 };
+
+// SWAP: the operands are given exchanged (A is the [N][K] one), so that a short N is the side held in
+// fragments; row and col are then C's column and row.
+template <class Cfg, bool SWAP>
+__global__ __launch_bounds__(Cfg::THREADS) void gemm_bf16_skinny(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
+                                                                 void* __restrict__ C, float* __restrict__ pre, int M, int N,
+                                                                 int K, int kind, int epi, int c_dtype,
+                                                                 uint16_t* __restrict__ ctr) {
+  __shared__ __attribute__((aligned(16))) char smem[Cfg::LDS_BYTES];
+  const int cm = SWAP ? N : M, cn = SWAP ? M : N;  // C's extents
+  const unsigned tiles_n = (N + Cfg::BN - 1) / Cfg::BN;
+  skinny_gemm<Cfg>(reinterpret_cast<const char*>(A), reinterpret_cast<const char*>(B), M, N, 2 * K,
+                   static_cast<int>(blockIdx.x / tiles_n) * Cfg::BM, static_cast<int>(blockIdx.x % tiles_n) * Cfg::BN, smem, [&](int i, int j, float v) {
+                     const int row = SWAP ? j : i, col = SWAP ? i : j;
+                     if (kind == kSkinnyForward) bf16_epilogue<0>(v, row, col, cm, cn, C, pre, epi, c_dtype, ctr);
+                     else if (kind == kSkinnyGeluBwd) bf16_epilogue<1>(v, row, col, cm, cn, C, pre, epi, c_dtype, ctr);
+                     else if (kind == kSkinnyMul) bf16_epilogue<2>(v, row, col, cm, cn, C, pre, epi, c_dtype, ctr);
+                     else bf16_epilogue<0, true>(v, row, col, cm, cn, C, pre, epi, c_dtype, ctr);
+                   });
+}
+
+// Whether a product takes gemm_skinny.h: a side below 128, which gives the 128-wide tiles at most one
+// row of blocks, while the blocks of 64 x 32 come to at most two per CU.  The same for every operand
+// form, so all give the same bits.  Packed [M][4096] x [4096][4096], us, weights rotating, tiles
+// before: M = 1 42.7 -> 7.4, 8 43.2 -> 8.2, 32 45.3 -> 11.4, 64 47.8 -> 18.5, 127 52.6 -> 19.6;
+// row-major [127] 39.8 -> 25.1, [300][1000] x [10] 17.8 -> 4.7.  A block reads its whole A side (43
+// GB/s a CU from L2), so four blocks per CU lose: [127][4096] x [16384] 95 against 59.
+bool skinny_runs(int64_t M, int64_t N, int64_t K) {
+  const int64_t s = M < N ? M : N, l = M < N ? N : M;
+  return s < 128 && (s <= 32 || ((s + 63) / 64) * ((l + 31) / 32) <= 512) && s * K >= 8 && gemm_config_override() < 0;
+}
+
+template <SkinnyForm FORM, bool SWAP>
+int launch_skinny_form(const uint16_t* A, const uint16_t* B, void* C, float* pre, int M, int N, int K, int kind, int epi, int ct,
+                       hipStream_t s, uint16_t* ctr) {
+  return skinny_dispatch<Mfma16Bf16, FORM>(M, N, int64_t{2} * K, [&](auto cfg) {
+    using Cfg = decltype(cfg);
+    const int64_t blocks = ((int64_t{N} + Cfg::BN - 1) / Cfg::BN) * ((int64_t{M} + Cfg::BM - 1) / Cfg::BM);
+    if (blocks > 0x7fffffff) return fail(VDSL_ERR_UNSUPPORTED, "GEMM: too many tiles");
+    const dim3 g(static_cast<unsigned>(blocks));
+    hipLaunchKernelGGL((gemm_bf16_skinny<Cfg, SWAP>), g, dim3(Cfg::THREADS), 0, s, A, B, C, pre, M, N, K, kind,
+                       epi & ~kEpiStreamOut, ct, ctr);
+    return check_launch("gemm_bf16_skinny");
+  });
+}
+
+int launch_skinny(bool packed, const uint16_t* A, const uint16_t* B, void* C, float* pre, int M, int N, int K, int kind, int epi,
+                  int ct, hipStream_t s, uint16_t* ctr) {
+  if (packed) return launch_skinny_form<kSkinnyPacked, false>(A, B, C, pre, M, N, K, kind, epi, ct, s, ctr);
+  if (M <= N) return launch_skinny_form<kSkinnyRows, false>(A, B, C, pre, M, N, K, kind, epi, ct, s, ctr);
+  return launch_skinny_form<kSkinnyRows, true>(B, A, C, pre, N, M, K, kind, epi, ct, s, ctr);
+}
+
 // ---- packed-weight form (gemm_bpk.h main loop): B in MFMA fragment order, A through LDS --------
 // For constant weights (forward GEMMs on [out][in] weights): the weight is packed once and each
 // wave loads its B fragments straight into registers.  Same k-steps in the same order with the same
@@ -636,6 +694,8 @@ int choose_config(int64_t M, int64_t N, int64_t K) {
 
 int launch_nt(const uint16_t* A, const uint16_t* B, void* C, float* pre, int M, int N, int K, int epi, int ct, hipStream_t s,
               uint16_t* ctr = nullptr) {
+  if (skinny_runs(M, N, K))
+    return launch_skinny(false, A, B, C, pre, M, N, K, epi == kEpiGeluBwd ? kSkinnyGeluBwd : kSkinnyForward, epi, ct, s, ctr);
   if (K % 8 != 0) {
     const int64_t blocks = (static_cast<int64_t>(M) * N + 255) / 256;
     hipLaunchKernelGGL(gemm_bf16_nt_simple, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, A, B, C, pre, M, N, K, epi, ct, ctr);
@@ -797,6 +857,11 @@ extern "C" int vdsl_op_gemm_bf16_packed(vdsl_queue q, int64_t M, int64_t N, int6
   VDSL_TRY(check_buffer(q, C, nbytes(M, N, dtype_size(c_dtype)), "C", true));
   if (pre_act) VDSL_TRY(check_buffer(q, pre_act, nbytes(M, N, 4), "pre_act", true));
   if (M == 0 || N == 0) return VDSL_OK;
+  if (skinny_runs(M, N, K))
+    return launch_skinny(true, static_cast<const uint16_t*>(A->ptr), static_cast<const uint16_t*>(Bp->ptr), C->ptr,
+                         pre_act ? static_cast<float*>(pre_act->ptr) : nullptr, static_cast<int>(M), static_cast<int>(N),
+                         static_cast<int>(K), epilogue == VDSL_EPI_GELU_DERIV ? kSkinnyDeriv : kSkinnyForward, epilogue, c_dtype,
+                         q->stream, nullptr);
   const int64_t tiles = ((M + Pb0::BM - 1) / Pb0::BM) * ((N + Pb0::BN - 1) / Pb0::BN);
   auto* kern = epilogue == VDSL_EPI_GELU_DERIV ? gemm_bf16_bpk<Pb0, 0, true> : gemm_bf16_bpk<Pb0, 0, false>;
   hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(tiles)), dim3(Pb0::NT), 0, q->stream,
@@ -819,6 +884,10 @@ extern "C" int vdsl_op_gemm_bf16_gelu_bwd_packed(vdsl_queue q, int64_t M, int64_
   VDSL_TRY(check_buffer(q, da, nbytes(M, N, 2), "da", true));
   if (da_t) VDSL_TRY(check_buffer(q, da_t, nbytes(M, N, 2), "da_t", true));
   if (M == 0 || N == 0) return VDSL_OK;
+  if (skinny_runs(M, N, K))
+    return launch_skinny(true, static_cast<const uint16_t*>(A->ptr), static_cast<const uint16_t*>(Bp->ptr), da->ptr,
+                         static_cast<float*>(pre->ptr), static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), kSkinnyGeluBwd,
+                         kEpiGeluBwd, VDSL_BF16, q->stream, da_t ? static_cast<uint16_t*>(da_t->ptr) : nullptr);
   const int64_t tiles = ((M + Pb0::BM - 1) / Pb0::BM) * ((N + Pb0::BN - 1) / Pb0::BN);
   hipLaunchKernelGGL((gemm_bf16_bpk<Pb0, 1>), dim3(static_cast<unsigned>(tiles)), dim3(Pb0::NT), 0, q->stream,
                      static_cast<const uint16_t*>(A->ptr), static_cast<const uint16_t*>(Bp->ptr), da->ptr,
@@ -840,6 +909,10 @@ extern "C" int vdsl_op_gemm_bf16_mul_packed(vdsl_queue q, int64_t M, int64_t N, 
   VDSL_TRY(check_buffer(q, c, nbytes(M, N, 2), "c", true));
   if (c_t) VDSL_TRY(check_buffer(q, c_t, nbytes(M, N, 2), "c_t", true));
   if (M == 0 || N == 0) return VDSL_OK;
+  if (skinny_runs(M, N, K))
+    return launch_skinny(true, static_cast<const uint16_t*>(A->ptr), static_cast<const uint16_t*>(Bp->ptr), c->ptr,
+                         static_cast<float*>(g->ptr), static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), kSkinnyMul,
+                         kEpiGeluBwd, VDSL_BF16, q->stream, c_t ? static_cast<uint16_t*>(c_t->ptr) : nullptr);
   const int64_t tiles = ((M + Pb0::BM - 1) / Pb0::BM) * ((N + Pb0::BN - 1) / Pb0::BN);
   hipLaunchKernelGGL((gemm_bf16_bpk<Pb0, 2>), dim3(static_cast<unsigned>(tiles)), dim3(Pb0::NT), 0, q->stream,
                      static_cast<const uint16_t*>(A->ptr), static_cast<const uint16_t*>(Bp->ptr), c->ptr,

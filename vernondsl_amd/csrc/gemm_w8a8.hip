@@ -10,14 +10,15 @@
 // v_mfma_i32_32x32x32_i8 fragment is 16 int8 per lane (A[row = l%32][k = 16*(l/32) .. +15]) and
 // the accumulator layout is the f32 one.  This file adds the dequant epilogue and the split-K path.
 //
-// Narrow outputs (too few tiles to fill 256 CUs, e.g. the 1024-wide last layer at batch 512)
-// split K across blocks: each block adds its int32 partial tile into a zeroed int32 workspace
+// Products with a short side (a few rows of activations) run gemm_skinny.h.  Other narrow outputs
+// (too few tiles to fill 256 CUs, e.g. the 1024-wide last layer at batch 512) split K across blocks: each block adds its int32 partial tile into a zeroed int32 workspace
 // with atomics - integer addition is exact and order-independent, so the result is still
 // deterministic - and a second kernel applies the dequant epilogue.
 
 #include "gemm_bpk.h"
 #include "gemm_dma.h"
 #include "gemm_mfma.h"
+#include "gemm_skinny.h"
 
 namespace vdsl {
 namespace {
@@ -418,6 +419,49 @@ int launch_w8a8(const int8_t* a, const int8_t* b, const float* xs, const float* 
 }
 
 
+// ---- products with a short side (gemm_skinny.h) -----------------------------------------------------
+template <class Cfg, bool SWAP>
+__global__ __launch_bounds__(Cfg::THREADS) void gemm_w8a8_skinny(const int8_t* __restrict__ A, const int8_t* __restrict__ B,
+                                                                 const float* __restrict__ xs, const float* __restrict__ wsc,
+                                                                 void* __restrict__ y, int out_dtype, int relu,
+                                                                 int32_t* __restrict__ acc_out, int M, int N, int K) {
+  __shared__ __attribute__((aligned(16))) char smem[Cfg::LDS_BYTES];
+  const unsigned tiles_n = (N + Cfg::BN - 1) / Cfg::BN;
+  skinny_gemm<Cfg>(reinterpret_cast<const char*>(A), reinterpret_cast<const char*>(B), M, N, K,
+                   static_cast<int>(blockIdx.x / tiles_n) * Cfg::BM, static_cast<int>(blockIdx.x % tiles_n) * Cfg::BN, smem, [&](int i, int j, int32_t a) {
+                     const int row = SWAP ? j : i, col = SWAP ? i : j;
+                     const size_t o = static_cast<size_t>(row) * (SWAP ? M : N) + col;
+                     if (acc_out) acc_out[o] = a;
+                     store_y(y, out_dtype, o, dequant(a, xs[row], wsc[col], relu));
+                   });
+}
+
+// Whether a product takes gemm_skinny.h: a short side of at most `most_rows`, or below 128 with K up
+// to `most_k` (a block reads its whole A side, the split-K tiles a part of it), and at most two blocks
+// of 64 x 32 per CU.  Packed, us, weights rotating, tiles before: [8][8192] x [8192] 24.5 -> 13.1, [32]
+// 24.7 -> 15.4, [8][8192] x [1024] 12.6 -> 6.7, [127][2048] x [2048] 9.5 -> 7.4; but [64][8192] x [1024]
+// 12.9 -> 18.4, [127][8192] x [8192] 28.9 -> 40.0: 32 rows or K of 2048.  Row-major: [64][2000] x [2000]
+// 10.7 -> 6.6, [8][8192] x [8192] 18.2 -> 16.3, [100][4096] x [4096] 14.4 either way: 64 rows or 4096.
+bool skinny_runs(int64_t M, int64_t N, int64_t K, int64_t most_rows, int64_t most_k) {
+  const int64_t s = M < N ? M : N, l = M < N ? N : M;
+  return s < 128 && (s <= most_rows || K <= most_k) && (s <= 32 || ((s + 63) / 64) * ((l + 31) / 32) <= 512) && K >= 16 &&
+         gemm_config_override() < 0;
+}
+
+template <SkinnyForm FORM, bool SWAP>
+int launch_skinny(const int8_t* a, const int8_t* b, const float* xs, const float* wsc, void* y, int out_dtype, int relu,
+                  int32_t* ao, int m, int n, int k, hipStream_t s) {
+  return skinny_dispatch<Mfma16I8, FORM>(m, n, k, [&](auto cfg) {
+    using Cfg = decltype(cfg);
+    const int64_t blocks = ((int64_t{n} + Cfg::BN - 1) / Cfg::BN) * ((int64_t{m} + Cfg::BM - 1) / Cfg::BM);
+    if (blocks > 0x7fffffff) return fail(VDSL_ERR_UNSUPPORTED, "GEMM: too many tiles");
+    const dim3 g(static_cast<unsigned>(blocks));
+    hipLaunchKernelGGL((gemm_w8a8_skinny<Cfg, SWAP>), g, dim3(Cfg::THREADS), 0, s, a, b, xs, wsc, y, out_dtype, relu, ao, m, n,
+                       k);
+    return check_launch("gemm_w8a8_skinny");
+  });
+}
+
 // ---- packed-weight GEMM (gemm_bpk.h main loop) ------------------------------------------------
 // Weights in fragment order (bpk_pack_kernel), activations row-major through LDS.  A launch of
 // tiles * S blocks: block (tile, z) covers K bytes [z K/S, (z+1) K/S) of its tile.  With S == 1 the
@@ -748,6 +792,10 @@ extern "C" int vdsl_op_gemm_w8a8(vdsl_queue q, int64_t M, int64_t N, int64_t K, 
   const auto* b = static_cast<const int8_t*>(w->ptr);
   const auto* xs = static_cast<const float*>(x_scale->ptr);
   const auto* wsc = static_cast<const float*>(w_scale->ptr);
+  if (skinny_runs(M, N, K, 64, 4096)) {
+    if (m <= n) return launch_skinny<kSkinnyRows, false>(a, b, xs, wsc, y->ptr, out_dtype, relu, ao, m, n, k, q->stream);
+    return launch_skinny<kSkinnyRows, true>(b, a, xs, wsc, y->ptr, out_dtype, relu, ao, n, m, k, q->stream);
+  }
   if (split == 1) return launch_w8a8(a, b, xs, wsc, y->ptr, out_dtype, relu, ao, nullptr, m, n, k, 1, q->stream);
   VDSL_TRY(vdsl_buffer_fill_u32(q, workspace, 0, static_cast<size_t>(M) * N * 4, 0u));
   int32_t* wacc = static_cast<int32_t*>(workspace->ptr);
@@ -818,6 +866,8 @@ static int packed_launch(vdsl_queue q, const BpkPlan& p, int64_t M, int64_t N, i
   const auto* xs = static_cast<const float*>(x_scale->ptr);
   const auto* wsc = static_cast<const float*>(w_scale->ptr);
   const int m = static_cast<int>(M), n = static_cast<int>(N), k = static_cast<int>(K);
+  if (skinny_runs(M, N, K, 32, 2048) && g_bpk_plan.load(std::memory_order_relaxed) < 0)
+    return launch_skinny<kSkinnyPacked, false>(a, b, xs, wsc, y->ptr, out_dtype, relu, ao, m, n, k, q->stream);
   if (p.cfg == 0) return launch_bpk<P0>(p, a, b, xs, wsc, y->ptr, out_dtype, relu, ao, part, m, n, k, q->stream);
   if (p.cfg == 3) return launch_bpk<P3>(p, a, b, xs, wsc, y->ptr, out_dtype, relu, ao, part, m, n, k, q->stream);
   if (p.cfg == 4) return launch_bpk<P4>(p, a, b, xs, wsc, y->ptr, out_dtype, relu, ao, part, m, n, k, q->stream);
