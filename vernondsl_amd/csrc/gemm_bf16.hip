@@ -4,17 +4,19 @@
 // autodiff-generated backward).
 //
 // Native layout "NT": C[m][n] = sum_k A[m][k] * B[n][k], both operands K-contiguous (B is a
-// weight in [out][in] form).  The other layouts are reduced to it by transposing the strided
-// operand into caller-provided workspace first (vdsl_gemm_bf16_workspace_bytes).  The main loop
-// (tiling, LDS double buffering, MFMA fragment layout, XCD-aware order) is gemm_mfma.h; this file
-// adds the epilogue (GELU / ReLU, optional f32 pre-activation, f32 or bf16 C) and the choice of
-// tile configuration per shape.
+// weight in [out][in] form).  The other layouts are read as stored (gemm_any.h, gemm_dma.h's K-major
+// forms) or, large, reduced to it by transposing the strided operand into caller-provided workspace
+// first (vdsl_gemm_bf16_workspace_bytes).  The main loops are gemm_dma.h, gemm_bpk.h (packed
+// weights), gemm_skinny.h (a short side), gemm_any.h (any layout and extents) and gemm_mfma.h; this
+// file adds the epilogue (GELU / ReLU, optional f32 pre-activation, f32 or bf16 C) and the choice of
+// loop and tile configuration per shape.
 
 #include <atomic>
 #include <cstdlib>
 
 #include "gemm_mfma.h"
 #include "gemm_bpk.h"
+#include "gemm_any.h"
 #include "gemm_dma.h"
 #include "gemm_skinny.h"
 
@@ -474,6 +476,55 @@ __global__ __launch_bounds__(256) void gemm_bf16_nt_simple(const uint16_t* __res
   else static_cast<uint16_t*>(C)[idx] = f32_to_bf16(y);
 }
 
+// ---- operands as they are stored, any extents (gemm_any.h) -----------------------------------------
+template <class Cfg, bool BWD>
+__global__ __launch_bounds__(Cfg::NT) void gemm_bf16_any(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
+                                                         void* __restrict__ C, float* __restrict__ pre, int M, int N, int K,
+                                                         int epi, int c_dtype, uint16_t* __restrict__ ctr) {
+  __shared__ __attribute__((aligned(16))) char smem[Cfg::LDS_BYTES];
+  const int tiles_m = (M + Cfg::BM - 1) / Cfg::BM, tiles_n = (N + Cfg::BN - 1) / Cfg::BN;
+  int tm, tn;
+  tile_coords(xcd_remap(blockIdx.x, gridDim.x), tiles_m, tiles_n, tm, tn);
+  f32x16 acc[Cfg::FM][Cfg::FN];
+  any_mainloop<Cfg>(A, B, M, N, K, tm * Cfg::BM, tn * Cfg::BN, smem, acc);
+  bf16_store_tile<Cfg, BWD>(acc, tm * Cfg::BM, tn * Cfg::BN, M, N, C, pre, epi & ~kEpiStreamOut, c_dtype, ctr);
+}
+
+int64_t tiles64(int64_t M, int64_t N) { return ((M + 63) / 64) * ((N + 63) / 64); }
+
+// Both operands hold the 16 bytes that its loads take at least, and no configuration is forced.
+bool any_runs(int64_t M, int64_t N, int64_t K) { return M * K >= 8 && N * K >= 8 && gemm_config_override() < 0; }
+
+template <bool AKM, bool BKM>
+int launch_any_form(const uint16_t* A, const uint16_t* B, void* C, float* pre, int M, int N, int K, int epi, int ct, hipStream_t s,
+                    uint16_t* ctr) {
+  const auto go = [&](auto cfg) {
+    using Cfg = decltype(cfg);
+    const int64_t tiles = ((int64_t{M} + Cfg::BM - 1) / Cfg::BM) * ((int64_t{N} + Cfg::BN - 1) / Cfg::BN);
+    if (tiles > 0x7fffffff) return fail(VDSL_ERR_UNSUPPORTED, "GEMM: too many tiles");
+    if (epi == kEpiGeluBwd)
+      hipLaunchKernelGGL((gemm_bf16_any<Cfg, true>), dim3(static_cast<unsigned>(tiles)), dim3(Cfg::NT), 0, s, A, B, C, pre, M, N, K,
+                         epi, ct, ctr);
+    else
+      hipLaunchKernelGGL((gemm_bf16_any<Cfg, false>), dim3(static_cast<unsigned>(tiles)), dim3(Cfg::NT), 0, s, A, B, C, pre, M, N,
+                         K, epi, ct, ctr);
+    return check_launch("gemm_bf16_any");
+  };
+  // 64 x 64 tiles below 1024 of them (3000x1000x600 16.3 us against 19.3 with 128 x 128, 512^3 6.4 against
+  // 10.4), 128 x 128 from there on (2048^3 31.1 against 35.4, 4000x4000x2000 102 against 181).
+  if (tiles64(M, N) < 1024) return go(AnyConfig<64, 64, 2, 2, AKM, BKM>{});
+  return go(AnyConfig<128, 128, 2, 2, AKM, BKM>{});
+}
+
+// A stored [K][M] if ta, B stored [K][N] if !tb; any_runs(M, N, K).
+int launch_any(bool ta, bool tb, const uint16_t* A, const uint16_t* B, void* C, float* pre, int M, int N, int K, int epi, int ct,
+               hipStream_t s, uint16_t* ctr = nullptr) {
+  if (ta) return tb ? launch_any_form<true, false>(A, B, C, pre, M, N, K, epi, ct, s, ctr)
+                    : launch_any_form<true, true>(A, B, C, pre, M, N, K, epi, ct, s, ctr);
+  return tb ? launch_any_form<false, false>(A, B, C, pre, M, N, K, epi, ct, s, ctr)
+            : launch_any_form<false, true>(A, B, C, pre, M, N, K, epi, ct, s, ctr);
+}
+
 // ---- products with a short side (gemm_skinny.h) -----------------------------------------------------
 // Epilogue kinds of one kernel: the forward ones (`epi` selects it), the two backward ones and
 // VDSL_EPI_GELU_DERIV, as bf16_epilogue's template arguments.
@@ -696,6 +747,15 @@ int launch_nt(const uint16_t* A, const uint16_t* B, void* C, float* pre, int M, 
               uint16_t* ctr = nullptr) {
   if (skinny_runs(M, N, K))
     return launch_skinny(false, A, B, C, pre, M, N, K, epi == kEpiGeluBwd ? kSkinnyGeluBwd : kSkinnyForward, epi, ct, s, ctr);
+  // Row-major operands by gemm_any.h: rows that are not whole 16-byte units (one lane per output
+  // before: 300x784x1000 with K = 300, 303 us against 7), outputs of fewer than 512 tiles of 64 x 64
+  // (256 x 256 and 128-wide tiles leave CUs idle: 300x4096x4096 44.6 us against 36.3, 512^3 7.4 against
+  // 6.4; 2048^3, 1024 tiles, 30.6 against 31.1), 1024 where K has no 64-byte stages (1500x1500x1000 23.4
+  // against 19.1, 300x784x1000 20.8 against 11.6; 2000x4000x1000 31.7 against 33.0), and those where that
+  // loop takes its 256-wide tiles (4000x4000x2000 126 against 102).
+  if (any_runs(M, N, K) &&
+      (K % 8 != 0 || tiles64(M, N) < (K % 32 == 0 ? 512 : 1024) || (K % 32 != 0 && choose_config(M, N, K) == 13)))
+    return launch_any(false, true, A, B, C, pre, M, N, K, epi, ct, s, ctr);
   if (K % 8 != 0) {
     const int64_t blocks = (static_cast<int64_t>(M) * N + 255) / 256;
     hipLaunchKernelGGL(gemm_bf16_nt_simple, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, A, B, C, pre, M, N, K, epi, ct, ctr);
@@ -789,6 +849,14 @@ extern "C" int vdsl_op_gemm_bf16(vdsl_queue q, int32_t trans_a, int32_t trans_b,
     return launch_dma_kn(choose_config(M, N, K), a, b, C->ptr, pre, static_cast<int>(M), static_cast<int>(N),
                          static_cast<int>(K), epi, c_dtype, q->stream, ta);
   }
+  // Transposed operands read as stored (gemm_any.h) instead of transposing them into the workspace
+  // first (1000x784x300 TN 24.8 us against 7.2, 2048^3 40.2 against 31.1, 2000x4096x4096 94.2 against 92.7),
+  // but for outputs large enough that the direct-to-LDS tiles repay the transposes (4032x4096x2048 TN
+  // 87.0 against 97.6, 8000x8192x4096 522 against 657).
+  const bool large = K % 32 == 0 && ((M + 127) / 128) * ((N + 127) / 128) > 768;
+  if (any_runs(M, N, K) && (ta || !tb) && !large)
+    return launch_any(ta, tb, a, b, C->ptr, pre, static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), epi, c_dtype,
+                      q->stream);
   char* w = ws ? static_cast<char*>(workspace->ptr) : nullptr;
   if (ta) {  // A stored [K][M] -> [M][K]
     VDSL_TRY(launch_transpose(a, w, K, M, VDSL_BF16, q->stream));

@@ -47,12 +47,9 @@ struct __attribute__((packed, aligned(2))) Bytes16 {
 
 __device__ __forceinline__ u32x4 load16(const char* p) { return reinterpret_cast<const Bytes16*>(p)->v; }
 
-// The 16 bytes at byte offset `at` of a tensor of `size` >= 16 bytes, those past its end as 0 and
-// never read: lanes near the end load the tensor's last 16 bytes and shift them down.
-__device__ __forceinline__ u32x4 load16_to_end(const char* __restrict__ base, int64_t at, int64_t size) {
-  const int64_t last = size - 16, from = at < last ? at : last;
-  u32x4 v = load16(base + from);
-  const int w = at - from > 16 ? 16 : static_cast<int>(at - from), sh = 8 * (w & 3);
+// v shifted down by w (0..16) bytes, zeros entering at the top.
+__device__ __forceinline__ u32x4 shift_down(u32x4 v, int w) {
+  const int sh = 8 * (w & 3);
   uint32_t t[5] = {v[0], v[1], v[2], v[3], 0u};
 #pragma unroll
   for (int s = 1; s <= 4; ++s) {
@@ -64,6 +61,13 @@ __device__ __forceinline__ u32x4 load16_to_end(const char* __restrict__ base, in
 #pragma unroll
   for (int e = 0; e < 4; ++e) v[e] = static_cast<uint32_t>((static_cast<uint64_t>(t[e + 1]) << 32 | t[e]) >> sh);
   return v;
+}
+
+// The 16 bytes at byte offset `at` of a tensor of `size` >= 16 bytes, those past its end as 0 and
+// never read: lanes near the end load the tensor's last 16 bytes and shift them down.
+__device__ __forceinline__ u32x4 load16_to_end(const char* __restrict__ base, int64_t at, int64_t size) {
+  const int64_t last = size - 16, from = at < last ? at : last;
+  return shift_down(load16(base + from), at - from > 16 ? 16 : static_cast<int>(at - from));
 }
 
 // Bytes of v from `keep` on set to 0 (keep may be negative or past 16).
