@@ -169,6 +169,19 @@ __global__ __launch_bounds__(256) void mse_tile_vec(const float* __restrict__ y,
   store_pair_tile_transposed(tile, dy_t, rows, cols, r0, c0);
 }
 
+// A lane's 16 elements of two tensors, rows r, r + 4, ... of column c, all loaded before any is used
+// (rows and columns past the end repeat the last one; a branch around each load waits for it: the MSE
+// of [300][10] 7.1 us with it, 3.8 without).
+__device__ __forceinline__ void load_column(const float* __restrict__ p, const float* __restrict__ q, int64_t r, int64_t c,
+                                            int64_t rows, int64_t cols, float (&a)[16], float (&b)[16]) {
+#pragma unroll
+  for (int k = 0; k < 16; ++k) {
+    const int64_t o = (r + 4 * k < rows ? r + 4 * k : rows - 1) * cols + (c < cols ? c : cols - 1);
+    a[k] = p[o];
+    b[k] = q[o];
+  }
+}
+
 template <int ACT>
 __global__ __launch_bounds__(256) void act_bwd_kernel(const float* __restrict__ dh, const float* __restrict__ pre,
                                                       uint16_t* __restrict__ da, uint16_t* __restrict__ da_t,
@@ -176,13 +189,15 @@ __global__ __launch_bounds__(256) void act_bwd_kernel(const float* __restrict__ 
   __shared__ uint16_t tile[64][66];
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
   const int64_t r0 = static_cast<int64_t>(blockIdx.y) * 64, c0 = static_cast<int64_t>(blockIdx.x) * 64;
-#pragma unroll 4
+  const int64_t c = c0 + tx;
+  float g[16], x[16];
+  load_column(dh, pre, r0 + ty, c, rows, cols, g, x);
+#pragma unroll
   for (int p = 0; p < 16; ++p) {
-    const int64_t r = r0 + ty + 4 * p, c = c0 + tx;
+    const int64_t r = r0 + ty + 4 * p;
     if (r < rows && c < cols) {
-      const int64_t o = r * cols + c;
-      const uint16_t h = f32_to_bf16(act_bwd<ACT>(dh[o], pre[o]));
-      da[o] = h;
+      const uint16_t h = f32_to_bf16(act_bwd<ACT>(g[p], x[p]));
+      da[r * cols + c] = h;
       tile[ty + 4 * p][tx] = h;
     }
   }
@@ -204,15 +219,17 @@ __global__ __launch_bounds__(256) void mse_tile_kernel(const float* __restrict__
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
   const int64_t r0 = static_cast<int64_t>(blockIdx.y) * 64, c0 = static_cast<int64_t>(blockIdx.x) * 64;
   double s = 0.0;
-#pragma unroll 4
+  const int64_t c = c0 + tx;
+  float a[16], b[16];
+  load_column(y, t, r0 + ty, c, rows, cols, a, b);
+#pragma unroll
   for (int p = 0; p < 16; ++p) {
-    const int64_t r = r0 + ty + 4 * p, c = c0 + tx;
+    const int64_t r = r0 + ty + 4 * p;
     if (r < rows && c < cols) {
-      const int64_t o = r * cols + c;
-      const float d = y[o] - t[o];
+      const float d = a[p] - b[p];
       s += static_cast<double>(d) * static_cast<double>(d);
       const uint16_t h = f32_to_bf16(d * scale);
-      if (dy) dy[o] = h;
+      if (dy) dy[r * cols + c] = h;
       tile[ty + 4 * p][tx] = h;
     }
   }

@@ -476,6 +476,34 @@ __global__ __launch_bounds__(256) void gemm_bf16_nt_simple(const uint16_t* __res
   else static_cast<uint16_t*>(C)[idx] = f32_to_bf16(y);
 }
 
+// The GELU-backward epilogue per element with a 32-row block's loads of `pre` issued before the first is
+// used (clamped to the tensor; one load per element and branch waited for each in turn: 300x1000x10 10.0 us, 7.2 here).
+template <class Cfg>
+__device__ __forceinline__ void bf16_store_tile_bwd(const f32x16 (&acc)[Cfg::FM][Cfg::FN], int m0, int n0, int M, int N,
+                                                    void* __restrict__ C, const float* __restrict__ pre,
+                                                    uint16_t* __restrict__ ctr) {
+#pragma unroll
+  for (int i = 0; i < Cfg::FM; ++i) {
+    float x[Cfg::FN][16];
+#pragma unroll
+    for (int j = 0; j < Cfg::FN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        x[j][r] = pre[static_cast<size_t>(min(acc_row<Cfg>(m0, i, r), M - 1)) * N + min(acc_col<Cfg>(n0, j), N - 1)];
+#pragma unroll
+    for (int j = 0; j < Cfg::FN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int row = acc_row<Cfg>(m0, i, r), col = acc_col<Cfg>(n0, j);
+        const uint16_t h = f32_to_bf16(acc[i][j][r] * bwd_factor<1>(x[j][r]));
+        if (row < M && col < N) {
+          static_cast<uint16_t*>(C)[static_cast<size_t>(row) * N + col] = h;
+          if (ctr) ctr[static_cast<size_t>(col) * M + row] = h;
+        }
+      }
+  }
+}
+
 // ---- operands as they are stored, any extents (gemm_any.h) -----------------------------------------
 template <class Cfg, bool BWD>
 __global__ __launch_bounds__(Cfg::NT) void gemm_bf16_any(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
@@ -487,7 +515,8 @@ __global__ __launch_bounds__(Cfg::NT) void gemm_bf16_any(const uint16_t* __restr
   tile_coords(xcd_remap(blockIdx.x, gridDim.x), tiles_m, tiles_n, tm, tn);
   f32x16 acc[Cfg::FM][Cfg::FN];
   any_mainloop<Cfg>(A, B, M, N, K, tm * Cfg::BM, tn * Cfg::BN, smem, acc);
-  bf16_store_tile<Cfg, BWD>(acc, tm * Cfg::BM, tn * Cfg::BN, M, N, C, pre, epi & ~kEpiStreamOut, c_dtype, ctr);
+  if constexpr (BWD) bf16_store_tile_bwd<Cfg>(acc, tm * Cfg::BM, tn * Cfg::BN, M, N, C, pre, ctr);
+  else bf16_store_tile<Cfg, 0>(acc, tm * Cfg::BM, tn * Cfg::BN, M, N, C, pre, epi & ~kEpiStreamOut, c_dtype, ctr);
 }
 
 int64_t tiles64(int64_t M, int64_t N) { return ((M + 63) / 64) * ((N + 63) / 64); }
