@@ -48,8 +48,8 @@ def test_row_major(dev, q, M, N, K):
         t.free()
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 32, 256), (8, 96, 4096), (20, 8192, 256), (64, 544, 512), (100, 96, 512), (127, 32, 2304),
-                                   (300, 64, 2048), (2000, 96, 256)])
+@pytest.mark.parametrize("M,N,K", [(1, 32, 256), (8, 96, 4096), (20, 8192, 256), (32, 544, 512), (31, 96, 512), (127, 32, 2304),
+                                   (300, 32, 2048), (2000, 32, 256)])
 def test_packed_equals_row_major(dev, q, M, N, K):
     """Packed weights, with every epilogue, against the row-major form and the separate ops, bit for
     bit (K is split alike for all of them)."""
@@ -128,3 +128,34 @@ def test_nan_next_to_k_ends(dev, q):
         assert np.array_equal(nan, want)
         for t in (tx, ty, out):
             t.free()
+
+
+@pytest.mark.parametrize("M,N,K", [(33, 64, 256), (64, 1024, 512), (100, 96, 512), (130, 4096, 256), (300, 2080, 256), (500, 4096, 512),
+                                   (1000, 2048, 256), (2000, 64, 256)])
+def test_packed_tiles(dev, q, M, N, K):
+    """Every tile size of the packed product (32 x 64 to 128 x 256, whole and ragged) with every epilogue,
+    bit for bit against the row-major tiles and the separate ops."""
+    a, b = operands(M, N, K, M * 3 + N + K)
+    ta, tb, tbp = Tensor.from_numpy(dev, q, a, "bf16"), Tensor.from_numpy(dev, q, b, "bf16"), Tensor(dev, (N, K), "bf16")
+    kernels.pack_bf16_weights(q, tb, tbp)
+    f = [Tensor(dev, (M, N), "f32") for _ in range(4)]
+    h = [Tensor(dev, (M, N), "bf16") for _ in range(6)]
+    ht = [Tensor(dev, (N, M), "bf16") for _ in range(3)]
+    kernels.gemm_bf16(q, ta, tb, f[0], False, True)
+    kernels.gemm_bf16_packed(q, ta, tbp, f[1])
+    got = f[0].numpy(q)
+    af, bf = rng.bf16_to_f32(a).astype(np.float64), rng.bf16_to_f32(b).astype(np.float64)
+    assert np.all(np.abs(got - af @ bf.T) <= K * 2.0 ** -24 * (np.abs(af) @ np.abs(bf).T))
+    assert np.array_equal(got, f[1].numpy(q))
+    kernels.gemm_bf16(q, ta, tb, h[0], False, True, _lib.EPI_GELU, f[1])
+    kernels.gemm_bf16_packed(q, ta, tbp, h[1], _lib.EPI_GELU, f[2])
+    kernels.gemm_bf16_packed(q, ta, tbp, h[2], _lib.EPI_GELU_DERIV, f[3])
+    ref = h[0].numpy(q)
+    assert np.array_equal(f[2].numpy(q), got) and np.array_equal(h[1].numpy(q), ref) and np.array_equal(h[2].numpy(q), ref)
+    kernels.gelu_bwd(q, f[0], f[0], h[3], ht[0])
+    kernels.gemm_bf16_gelu_bwd(q, ta, tbp, f[0], h[4], ht[1], packed=True)
+    kernels.gemm_bf16_mul_packed(q, ta, tbp, f[3], h[5], ht[2])
+    for x, y in ((h[4], h[3]), (h[5], h[3]), (ht[1], ht[0]), (ht[2], ht[0])):
+        assert np.array_equal(x.numpy(q), y.numpy(q))
+    for t in [ta, tb, tbp] + f + h + ht:
+        t.free()

@@ -478,7 +478,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_nt_simple(const uint16_t* __res
 
 // The GELU-backward epilogue per element with a 32-row block's loads of `pre` issued before the first is
 // used (clamped to the tensor; one load per element and branch waited for each in turn: 300x1000x10 10.0 us, 7.2 here).
-template <class Cfg>
+template <class Cfg, int BWD>
 __device__ __forceinline__ void bf16_store_tile_bwd(const f32x16 (&acc)[Cfg::FM][Cfg::FN], int m0, int n0, int M, int N,
                                                     void* __restrict__ C, const float* __restrict__ pre,
                                                     uint16_t* __restrict__ ctr) {
@@ -495,7 +495,7 @@ __device__ __forceinline__ void bf16_store_tile_bwd(const f32x16 (&acc)[Cfg::FM]
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int row = acc_row<Cfg>(m0, i, r), col = acc_col<Cfg>(n0, j);
-        const uint16_t h = f32_to_bf16(acc[i][j][r] * bwd_factor<1>(x[j][r]));
+        const uint16_t h = f32_to_bf16(acc[i][j][r] * bwd_factor<BWD>(x[j][r]));
         if (row < M && col < N) {
           static_cast<uint16_t*>(C)[static_cast<size_t>(row) * N + col] = h;
           if (ctr) ctr[static_cast<size_t>(col) * M + row] = h;
@@ -515,7 +515,7 @@ __global__ __launch_bounds__(Cfg::NT) void gemm_bf16_any(const uint16_t* __restr
   tile_coords(xcd_remap(blockIdx.x, gridDim.x), tiles_m, tiles_n, tm, tn);
   f32x16 acc[Cfg::FM][Cfg::FN];
   any_mainloop<Cfg>(A, B, M, N, K, tm * Cfg::BM, tn * Cfg::BN, smem, acc);
-  if constexpr (BWD) bf16_store_tile_bwd<Cfg>(acc, tm * Cfg::BM, tn * Cfg::BN, M, N, C, pre, ctr);
+  if constexpr (BWD) bf16_store_tile_bwd<Cfg, 1>(acc, tm * Cfg::BM, tn * Cfg::BN, M, N, C, pre, ctr);
   else bf16_store_tile<Cfg, 0>(acc, tm * Cfg::BM, tn * Cfg::BN, M, N, C, pre, epi & ~kEpiStreamOut, c_dtype, ctr);
 }
 
@@ -579,15 +579,18 @@ __global__ __launch_bounds__(Cfg::THREADS) void gemm_bf16_skinny(const uint16_t*
                    });
 }
 
-// Whether a product takes gemm_skinny.h: a side below 128, which gives the 128-wide tiles at most one
-// row of blocks, while the blocks of 64 x 32 come to at most two per CU.  The same for every operand
-// form, so all give the same bits.  Packed [M][4096] x [4096][4096], us, weights rotating, tiles
-// before: M = 1 42.7 -> 7.4, 8 43.2 -> 8.2, 32 45.3 -> 11.4, 64 47.8 -> 18.5, 127 52.6 -> 19.6;
-// row-major [127] 39.8 -> 25.1, [300][1000] x [10] 17.8 -> 4.7.  A block reads its whole A side (43
-// GB/s a CU from L2), so four blocks per CU lose: [127][4096] x [16384] 95 against 59.
+// Whether a product takes gemm_skinny.h: a side of at most 32, or one below 128 whose long operand
+// cannot be packed, while the blocks of 64 x 32 come to at most two per CU.  The same for every operand
+// form, so all give the same bits.  us, operands rotating, packed [M][4096] x [4096][4096] with 128 x
+// 256 tiles before, here, and in 32 x 64 tiles: M = 1 42.7, 7.4; 8 43.2, 8.2; 20 44.5, 10.2, 15.4; 32
+// 45.3, 11.5, 14.2; 64 47.8, 18.5, 14.4; 127 52.6, 19.6, 16.4.  Row-major (tiles before, here): [127] 39.8,
+// 25.1; [300][1000] x [10] 17.8, 4.7.  A block reads its whole A side (43 GB/s a CU from L2), so four
+// blocks per CU lose: [127][4096] x [16384] 59 against 95.
 bool skinny_runs(int64_t M, int64_t N, int64_t K) {
   const int64_t s = M < N ? M : N, l = M < N ? N : M;
-  return s < 128 && (s <= 32 || ((s + 63) / 64) * ((l + 31) / 32) <= 512) && s * K >= 8 && gemm_config_override() < 0;
+  const bool packable = N % 32 == 0 && K % 256 == 0;
+  return (s <= 32 || (s < 128 && !packable && ((s + 63) / 64) * ((l + 31) / 32) <= 512)) && s * K >= 8 &&
+         gemm_config_override() < 0;
 }
 
 template <SkinnyForm FORM, bool SWAP>
@@ -617,6 +620,35 @@ int launch_skinny(bool packed, const uint16_t* A, const uint16_t* B, void* C, fl
 // MFMA as every other configuration, so the same results bit for bit.  Measured standalone on
 // 2048x4096x4096 (random bf16, f32 out): 61-63 us against 66-68 us for the direct-to-LDS kernel.
 using Pb0 = BpkConfig<MfmaBf16, 4, 2, 4, 3>;  // 128 x 256 blocks, 4 waves of 128 x 64
+// Smaller tiles for outputs that give 128 x 256 blocks to a part of the CUs.
+using Pb1 = BpkConfig<MfmaBf16, 4, 1, 4, 3>;  // 128 x 128 blocks, 4 waves of 128 x 32
+using Pb2 = BpkConfig<MfmaBf16, 2, 1, 4, 3>;  // 64 x 128 blocks, 4 waves of 64 x 32
+using Pb3 = BpkConfig<MfmaBf16, 2, 1, 2, 3>;  // 64 x 64 blocks, 2 waves of 64 x 32
+using Pb4 = BpkConfig<MfmaBf16, 1, 1, 2, 3>;  // 32 x 64 blocks, 2 waves of 32 x 32
+
+// Calls go(Cfg{}, tiles) with the tile of a packed product.  A CU takes in about 55 GB/s of operands
+// from its L2, so a launch lasts as long as the operand bytes of its busiest CU: rounds of tiles over
+// the 256 CUs times the tile's rows and columns; a smaller tile is taken where that is less by a tenth
+// or more.  K = 4096, N = 4096, us for 128 x 256 and the choice: M = 64 47.8, 14.4 (32 x 64); 128 40.6, 15.2
+// (32 x 64); 300 46.5, 26.3 (64 x 128); 512 51.5, 28.7 (64 x 128); 2048 65.9 (128 x 256; 128 x 128 78.7);
+// [2048][4096] x [1024] 41.7, 22.7 (64 x 128), [512][2048] x [2048] 23.5, 10.9 (64 x 64).
+template <class Go>
+int bpk_dispatch(int64_t M, int64_t N, Go&& go) {
+  const auto tiles = [&](int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+  const int sizes[5][2] = {{128, 256}, {128, 128}, {64, 128}, {64, 64}, {32, 64}};
+  int best = 0;
+  int64_t cost = 0;
+  for (int c = 0; c < 5; ++c) {
+    const int64_t t = (tiles(sizes[c][0], sizes[c][1]) + 255) / 256 * (sizes[c][0] + sizes[c][1]);
+    if (c == 0 || 10 * t <= 9 * cost) best = c, cost = t;
+  }
+  const int64_t n = tiles(sizes[best][0], sizes[best][1]);
+  if (best == 1) return go(Pb1{}, n);
+  if (best == 2) return go(Pb2{}, n);
+  if (best == 3) return go(Pb3{}, n);
+  if (best == 4) return go(Pb4{}, n);
+  return go(Pb0{}, n);
+}
 
 // BWD: the backward epilogues (1: vdsl_op_gemm_bf16_gelu_bwd_packed, C = da, pre an input, ctr =
 // da^T; 2: vdsl_op_gemm_bf16_mul_packed, the factor given); their LDS is enlarged so the whole wave
@@ -649,7 +681,10 @@ __global__ __launch_bounds__(Cfg::NT, 1) void gemm_bf16_bpk(const uint16_t* __re
                               m0, n0, smem, acc);
   static_assert(kLdsEpilogue<Cfg>, "the LDS-staged epilogue must fit the main loop's LDS");
   const bool whole = m0 + Cfg::BM <= M && n0 + Cfg::BN <= N && N % 4 == 0;
-  if constexpr (BWD != 0) {
+  if constexpr (BWD != 0 && Cfg::WTN % 64 != 0) {
+    bf16_store_tile_bwd<Cfg, BWD>(acc, m0, n0, M, N, C, pre, ctr);
+    return;
+  } else if constexpr (BWD != 0) {
     if (whole && (!ctr || M % 8 == 0)) {
       bf16_epilogue_bwd_lds<Cfg, bpk_bf16_smem<Cfg, true>(), BWD>(acc, m0, n0, M, N, C, pre, smem, ctr);
       return;
@@ -959,13 +994,15 @@ extern "C" int vdsl_op_gemm_bf16_packed(vdsl_queue q, int64_t M, int64_t N, int6
                          pre_act ? static_cast<float*>(pre_act->ptr) : nullptr, static_cast<int>(M), static_cast<int>(N),
                          static_cast<int>(K), epilogue == VDSL_EPI_GELU_DERIV ? kSkinnyDeriv : kSkinnyForward, epilogue, c_dtype,
                          q->stream, nullptr);
-  const int64_t tiles = ((M + Pb0::BM - 1) / Pb0::BM) * ((N + Pb0::BN - 1) / Pb0::BN);
-  auto* kern = epilogue == VDSL_EPI_GELU_DERIV ? gemm_bf16_bpk<Pb0, 0, true> : gemm_bf16_bpk<Pb0, 0, false>;
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(tiles)), dim3(Pb0::NT), 0, q->stream,
-                     static_cast<const uint16_t*>(A->ptr), static_cast<const uint16_t*>(Bp->ptr), C->ptr,
-                     pre_act ? static_cast<float*>(pre_act->ptr) : nullptr, static_cast<int>(M), static_cast<int>(N),
-                     static_cast<int>(K), epilogue | (stream_out(C, epilogue, c_dtype) ? kEpiStreamOut : 0), c_dtype, nullptr);
-  return check_launch("gemm_bf16_bpk");
+  return bpk_dispatch(M, N, [&](auto cfg, int64_t tiles) {
+    using Cfg = decltype(cfg);
+    auto* kern = epilogue == VDSL_EPI_GELU_DERIV ? gemm_bf16_bpk<Cfg, 0, true> : gemm_bf16_bpk<Cfg, 0, false>;
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(tiles)), dim3(Cfg::NT), 0, q->stream,
+                       static_cast<const uint16_t*>(A->ptr), static_cast<const uint16_t*>(Bp->ptr), C->ptr,
+                       pre_act ? static_cast<float*>(pre_act->ptr) : nullptr, static_cast<int>(M), static_cast<int>(N),
+                       static_cast<int>(K), epilogue | (stream_out(C, epilogue, c_dtype) ? kEpiStreamOut : 0), c_dtype, nullptr);
+    return check_launch("gemm_bf16_bpk");
+  });
 }
 
 extern "C" int vdsl_op_gemm_bf16_gelu_bwd_packed(vdsl_queue q, int64_t M, int64_t N, int64_t K, vdsl_buffer A,
@@ -985,12 +1022,14 @@ extern "C" int vdsl_op_gemm_bf16_gelu_bwd_packed(vdsl_queue q, int64_t M, int64_
     return launch_skinny(true, static_cast<const uint16_t*>(A->ptr), static_cast<const uint16_t*>(Bp->ptr), da->ptr,
                          static_cast<float*>(pre->ptr), static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), kSkinnyGeluBwd,
                          kEpiGeluBwd, VDSL_BF16, q->stream, da_t ? static_cast<uint16_t*>(da_t->ptr) : nullptr);
-  const int64_t tiles = ((M + Pb0::BM - 1) / Pb0::BM) * ((N + Pb0::BN - 1) / Pb0::BN);
-  hipLaunchKernelGGL((gemm_bf16_bpk<Pb0, 1>), dim3(static_cast<unsigned>(tiles)), dim3(Pb0::NT), 0, q->stream,
-                     static_cast<const uint16_t*>(A->ptr), static_cast<const uint16_t*>(Bp->ptr), da->ptr,
-                     static_cast<float*>(pre->ptr), static_cast<int>(M), static_cast<int>(N), static_cast<int>(K),
-                     kEpiGeluBwd, VDSL_BF16, da_t ? static_cast<uint16_t*>(da_t->ptr) : nullptr);
-  return check_launch("gemm_bf16_bpk<gelu_bwd>");
+  return bpk_dispatch(M, N, [&](auto cfg, int64_t tiles) {
+    using Cfg = decltype(cfg);
+    hipLaunchKernelGGL((gemm_bf16_bpk<Cfg, 1>), dim3(static_cast<unsigned>(tiles)), dim3(Cfg::NT), 0, q->stream,
+                       static_cast<const uint16_t*>(A->ptr), static_cast<const uint16_t*>(Bp->ptr), da->ptr,
+                       static_cast<float*>(pre->ptr), static_cast<int>(M), static_cast<int>(N), static_cast<int>(K),
+                       kEpiGeluBwd, VDSL_BF16, da_t ? static_cast<uint16_t*>(da_t->ptr) : nullptr);
+    return check_launch("gemm_bf16_bpk<gelu_bwd>");
+  });
 }
 
 extern "C" int vdsl_op_gemm_bf16_mul_packed(vdsl_queue q, int64_t M, int64_t N, int64_t K, vdsl_buffer A, vdsl_buffer Bp,
@@ -1010,12 +1049,14 @@ extern "C" int vdsl_op_gemm_bf16_mul_packed(vdsl_queue q, int64_t M, int64_t N, 
     return launch_skinny(true, static_cast<const uint16_t*>(A->ptr), static_cast<const uint16_t*>(Bp->ptr), c->ptr,
                          static_cast<float*>(g->ptr), static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), kSkinnyMul,
                          kEpiGeluBwd, VDSL_BF16, q->stream, c_t ? static_cast<uint16_t*>(c_t->ptr) : nullptr);
-  const int64_t tiles = ((M + Pb0::BM - 1) / Pb0::BM) * ((N + Pb0::BN - 1) / Pb0::BN);
-  hipLaunchKernelGGL((gemm_bf16_bpk<Pb0, 2>), dim3(static_cast<unsigned>(tiles)), dim3(Pb0::NT), 0, q->stream,
-                     static_cast<const uint16_t*>(A->ptr), static_cast<const uint16_t*>(Bp->ptr), c->ptr,
-                     static_cast<float*>(g->ptr), static_cast<int>(M), static_cast<int>(N), static_cast<int>(K),
-                     kEpiGeluBwd, VDSL_BF16, c_t ? static_cast<uint16_t*>(c_t->ptr) : nullptr);
-  return check_launch("gemm_bf16_bpk<mul>");
+  return bpk_dispatch(M, N, [&](auto cfg, int64_t tiles) {
+    using Cfg = decltype(cfg);
+    hipLaunchKernelGGL((gemm_bf16_bpk<Cfg, 2>), dim3(static_cast<unsigned>(tiles)), dim3(Cfg::NT), 0, q->stream,
+                       static_cast<const uint16_t*>(A->ptr), static_cast<const uint16_t*>(Bp->ptr), c->ptr,
+                       static_cast<float*>(g->ptr), static_cast<int>(M), static_cast<int>(N), static_cast<int>(K),
+                       kEpiGeluBwd, VDSL_BF16, c_t ? static_cast<uint16_t*>(c_t->ptr) : nullptr);
+    return check_launch("gemm_bf16_bpk<mul>");
+  });
 }
 
 extern "C" int vdsl_op_gemm_bf16_mse_packed(vdsl_queue q, int64_t M, int64_t N, int64_t K, vdsl_buffer A, vdsl_buffer Bp,
