@@ -1,0 +1,46 @@
+"""Reductions over a grid (histograms, sums) whose blocks go through bands of 8 or 16 rows, on grids of
+one band, of a band and one row, of ragged columns, and of several bands a block.  int32 targets are
+exact in any order; f32 targets of small dyadic values too (every partial sum is a multiple of 2^-4
+below 2^20)."""
+import numpy as np
+import pytest
+
+from vernondsl_amd import kernels, pixprog as pp
+from vernondsl_amd.rhi import Tensor
+
+pytestmark = pytest.mark.gpu
+
+
+def program(bins, n, dtype, store):
+    """target k < n: [0][floor(x * bins) + k] += k + 1 (an add past the last bin is dropped); the last
+    target: a sum of x at a constant index; with store, out = x."""
+    b = pp.Builder()
+    x = b.load(0)
+    at = b.op("floor", b.op("mul", x, float(bins)))
+    fx = [b.scatter_add(1 + k, 0.0, b.op("add", at, float(k)) if k else at, float(k + 1)) for k in range(n)]
+    fx.append(b.scatter_add(1 + n, 0.0, 0.0, x))
+    return pp.compile_program(b, out=x if store else None, effects=fx, in_dtypes=[pp.F32] + [dtype] * n + [pp.F32],
+                              in_extents=[None] + [(1, bins)] * n + [(1, 1)])
+
+
+@pytest.mark.parametrize("store", [False, True])
+@pytest.mark.parametrize("n, dtype", [(1, pp.I32), (2, pp.I32), (3, pp.I32), (1, pp.F32), (5, pp.I32)])
+@pytest.mark.parametrize("ni, nj", [(1, 1), (15, 255), (16, 256), (17, 257), (33, 64), (64, 1000), (1500, 1027)])
+def test_bands(dev, q, ni, nj, n, dtype, store):
+    bins = 100
+    x = (np.random.default_rng(ni + nj + n).integers(-2, 18, (ni, nj)) / 16.0).astype(np.float32)  # some outside [0, 1)
+    at = np.floor(x.astype(np.float64) * bins).astype(int)
+    tx, out = Tensor.from_numpy(dev, q, x), Tensor(dev, (ni, nj), "f32") if store else None
+    ts = [Tensor.from_numpy(dev, q, np.full((1, bins), k, np.int32 if dtype == pp.I32 else np.float32)) for k in range(n)]
+    total = Tensor.from_numpy(dev, q, np.zeros((1, 1), np.float32))
+    kernels.pixel_program(q, program(bins, n, dtype, store), [tx] + ts + [total], out, grid=(ni, nj))
+    for k, t in enumerate(ts):
+        e = (at + k)[(at + k >= 0) & (at + k < bins)]
+        want = k + (k + 1) * np.bincount(e, minlength=bins)
+        assert np.array_equal(t.numpy(q).astype(np.int64)[0], want)
+    assert np.abs(x).sum(dtype=np.float64) < 2 ** 20  # multiples of 2^-4 below 2^20: 24 bits, every sum exact
+    assert total.numpy(q)[0, 0] == x.sum(dtype=np.float64)
+    if store:
+        assert np.array_equal(out.numpy(q), x)
+    for t in [tx, total] + ts + ([out] if store else []):
+        t.free()

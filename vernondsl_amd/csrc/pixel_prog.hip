@@ -9,6 +9,7 @@
 
 #include <algorithm>
 #include <cstddef>
+#include <cmath>
 #include <cstdlib>
 #include <mutex>
 #include <string>
@@ -124,38 +125,82 @@ int privatized(const vdsl_pixel_program& p, const std::vector<char>& flags, int 
   return static_cast<int>(own);
 }
 
-// Rows per block in the row mapping (each thread evaluates that many pixels of its column, then
-// stores them).  Measured on 8192^2 f32 (graph replays, one box): y = 2x + 1 runs best with 4
-// (88.2 us; 2, 6, 8, 12, 16 rows: 87-97% of that rate), the clamped five-point stencil of
-// examples/heat.py with 8 (95.7 us; 6: 95.9, 10: 99.1, 12: 99.6-99.9, 4: 103.0, 16: 107.5).  A
-// program that stores nothing and adds only at constant indices (a reduction such as
-// `total[None] += x[i, j]`) adds once per block, and those adds to one element are serialised
-// (~13 ns each): 64 rows (the sum of an 8192^2 field: 834 / 420 / 214 us with 4 / 8 / 16 rows);
-// so does one whose other adds go to per-block copies in LDS (their flush is per block too).
-// VDSL_PIX_ROWS=r (1..64) overrides the choice, for tuning sweeps.
-int rows_per_block(const vdsl_pixel_program& p, const std::vector<char>& flags, const int32_t* priv) {
-  if (const char* e = std::getenv("VDSL_PIX_ROWS")) {  // tuning sweeps: rows per block, 1..64
-    const int r = std::atoi(e);
-    if (r >= 1 && r <= 64) return r;
-  }
+// Whether a program stores nothing and makes all its adds at constant indices or into per-block
+// copies in LDS (a reduction such as `total[None] += x[i, j]`, a histogram): its blocks add to memory
+// once each, at their end.
+bool is_reduction(const vdsl_pixel_program& p, const std::vector<char>& flags, const int32_t* priv) {
   const int total = p.n_pre + p.n_test + p.n_body + p.n_post;
-  bool gathers = false, reduction = p.out_kind == VDSL_PIX_OUT_NONE;
-  for (int pc = 0; pc < total; ++pc) {
-    gathers |= p.code[pc].op == VDSL_PIX_LOAD_AT;
+  bool reduction = p.out_kind == VDSL_PIX_OUT_NONE;
+  for (int pc = 0; pc < total; ++pc)
     if (scatter_op(p.code[pc].op) && ((!(flags[pc] & 4) && !priv[p.code[pc].a]) || p.code[pc].op == VDSL_PIX_STORE_AT))
       reduction = false;
-  }
-  return reduction ? 64 : gathers ? 8 : 4;
+  return reduction;
 }
 
-// Blocks of rows_per_block rows x 256 pixels for programs whose pixels all do the same work (no
+// VDSL_PIX_ROWS=r (1..64) overrides the rows per block, for tuning sweeps; 0 without it.
+int rows_override() {
+  const char* e = std::getenv("VDSL_PIX_ROWS");
+  const int r = e ? std::atoi(e) : 0;
+  return r >= 1 && r <= 64 ? r : 0;
+}
+
+// Rows a thread evaluates together in the row mapping (a pixel of its column in each, then the
+// stores or the adds).  Measured on 8192^2 f32 (graph replays, one box): y = 2x + 1 runs best with 4
+// (88.2 us; 2, 6, 8, 12, 16 rows: 87-97% of that rate), the clamped five-point stencil of
+// examples/heat.py with 8 (95.7 us; 6: 95.9, 10: 99.1, 12: 99.6-99.9, 4: 103.0, 16: 107.5).  A
+// reduction goes through bands of 16 where that takes few registers (a 256-bin histogram of 8192^2
+// 63.8 us, bands of 8 74.8), else of 8.
+int rows_per_block(const vdsl_pixel_program& p, const std::vector<char>& flags, bool reduction) {
+  const int r = rows_override();
+  if (r) return reduction ? std::min(r, 8) : r;
+  const int total = p.n_pre + p.n_test + p.n_body + p.n_post;
+  bool gathers = false;
+  int adds = 0;  // at per-pixel indices, held for all rows of a band (PixPending)
+  for (int pc = 0; pc < total; ++pc) {
+    gathers |= p.code[pc].op == VDSL_PIX_LOAD_AT;
+    adds += scatter_op(p.code[pc].op) && !(flags[pc] & 4);
+  }
+  if (reduction) return total <= 16 && adds <= 2 && !p.loop ? 16 : 8;
+  return gathers ? 8 : 4;
+}
+
+// Blocks of rows x 256 pixels for programs whose pixels all do the same work (no
 // escape loop), while the row count fits the grid's y extent; 16x16 patches otherwise.  0 for
 // the patches.
-int row_mapping(const vdsl_pixel_program& p, const std::vector<char>& flags, const int32_t* priv, int ni) {
+int row_mapping(const vdsl_pixel_program& p, const std::vector<char>& flags, bool reduction, int ni) {
   // never more rows per block than the grid has: a 1-D field is a grid of one row, whose blocks
   // would otherwise run their loops for rows that do not exist
-  const int rows = std::min(rows_per_block(p, flags, priv), std::max(ni, 1));
+  const int rows = std::min(rows_per_block(p, flags, reduction), std::max(ni, 1));
   return !(p.loop && p.test != VDSL_PIX_TEST_NONE) && (ni + rows - 1) / rows <= 65535 ? rows : 0;
+}
+
+// Bands of `rows` rows per block of a reduction.  Adds of many blocks to one element are serialised
+// (~13 ns each) while few blocks leave CUs and loads in flight short, so the best count grows as the
+// root of the pixels.  us with blocks of 64 rows (their adds one by one), and 256, 512, 768, 1024, 2048
+// blocks: 1885x5071, 256 bins 35.2; 25.6, 21.6, 22.8, 24.1, 29.9; 2603x6098, 369 bins 42.7; 38.6, 27.7,
+// 28.4, 30.9, 46.5; 8192x8192, 256 bins 129.0; 139, 81.8, 69.1, 63.8, 73.8.  Small grids had few
+// blocks: 777x1460, 1009 bins 16.2, here 11.2 (its two launches take about 10 from the host).
+// f32 sums keep 64 rows a block, and with them the lengths of the chains they are added in, and so do
+// programs with more adds than PixPending holds.  Where int32 adds are wave-uniform (made row by row, as
+// many whatever the block's rows), the block's waves wait on each: one band while that gives at most 4096
+// blocks, else at least 1024 blocks.  Row sums, blocks of 64 rows and here: 1024x1024 29.1, 9.6 us; 2000x5000
+// 42.1, 24.5 (420 blocks 62.7); 8192x8192 219, 209 (one band, whose LDS copies cost more: 259).
+int reduction_bands(const vdsl_pixel_program& p, const std::vector<char>& flags, int rows, int ni, int nj) {
+  if (const int r = rows_override()) return (r + rows - 1) / rows;
+  const int total = p.n_pre + p.n_test + p.n_body + p.n_post;
+  bool sums = false, uniform = false;
+  int pending = 0;
+  for (int pc = 0; pc < total; ++pc) {
+    if (!scatter_op(p.code[pc].op)) continue;
+    sums |= p.code[pc].op == VDSL_PIX_ATOMIC_ADD && p.in_dtypes[p.code[pc].a] != VDSL_I32;
+    uniform |= !(flags[pc] & 4) && (flags[pc] & 3) == 3;
+    pending += !(flags[pc] & 4);
+  }
+  if (sums || pending * rows > 32) return (std::min(64, ni) + rows - 1) / rows;
+  const int64_t units = ((nj + 255) / 256) * static_cast<int64_t>((ni + rows - 1) / rows);
+  if (uniform) return units <= 4096 ? 1 : static_cast<int>(std::min<int64_t>(units / 1024, ni));
+  const double blocks = std::max(256.0, std::sqrt(static_cast<double>(ni) * nj) / 8);
+  return static_cast<int>(std::min(std::max(1.0, units / blocks + 0.5), static_cast<double>(ni)));
 }
 
 // Registers an instruction reads (a, b, c as the opcode uses them).
@@ -250,7 +295,7 @@ struct Plan {
   std::vector<char> flags;
   int32_t priv[VDSL_PIX_MAX_INPUTS] = {}, priv_off[VDSL_PIX_MAX_INPUTS] = {};
   int32_t priv_total = 0;
-  int rows = 0;
+  int rows = 0, bands = 1;
 };
 
 Plan make_plan(const vdsl_pixel_program& p, int n_inputs, int ni, int nj) {
@@ -261,7 +306,9 @@ Plan make_plan(const vdsl_pixel_program& p, int n_inputs, int ni, int nj) {
     pl.priv_off[k] = pl.priv_total;
     pl.priv_total += pl.priv[k];
   }
-  pl.rows = row_mapping(p, pl.flags, pl.priv, ni);
+  const bool reduction = is_reduction(p, pl.flags, pl.priv);
+  pl.rows = row_mapping(p, pl.flags, reduction, ni);
+  if (reduction && pl.rows) pl.bands = std::min(reduction_bands(p, pl.flags, pl.rows, ni, nj), (ni + pl.rows - 1) / pl.rows);
   return pl;
 }
 
@@ -324,7 +371,7 @@ std::string program_source(const vdsl_pixel_program& p, const Plan& pl, int n_in
 // the compiled-program cache, whose entries stay for the process.
 struct Launch {
   const JitKernels* k = nullptr;
-  int rows = 0;
+  int rows = 0, bands = 1;
 };
 std::mutex g_launch_mu;
 std::unordered_map<std::string, Launch> g_launches;
@@ -409,12 +456,14 @@ extern "C" int vdsl_op_pixel_program(vdsl_queue q, int32_t ni, int32_t nj, const
       return fail(VDSL_ERR_CAPTURE, "pixel program: not compiled yet; run it once before recording a graph");
     VDSL_TRY(st);
     ln.rows = pl.rows;
+    ln.bands = pl.bands;
     keep_launch(key, ln);
   }
   const JitKernels* k = ln.k;
   void* o = p.out_kind == VDSL_PIX_OUT_NONE ? nullptr : out->ptr;
   void* args[] = {&rt, &in, &o, &ni, &nj};
-  const int rows = ln.rows;
+  rt.bands = ln.bands;
+  const int rows = ln.rows * ln.bands;  // of a block
   const unsigned gx = rows ? static_cast<unsigned>((nj + 255) / 256) : static_cast<unsigned>((nj + 15) / 16);
   const unsigned gy = rows ? static_cast<unsigned>((ni + rows - 1) / rows) : static_cast<unsigned>((ni + 15) / 16);
   return check_hip(hipModuleLaunchKernel(k->fn[0], gx, gy, 1, 256, 1, 1, 0, q->stream, args, nullptr),

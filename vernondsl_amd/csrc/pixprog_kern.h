@@ -28,6 +28,7 @@ namespace vdsl {
 struct PixRt {
   float imm[VDSL_PIX_MAX_INSTR];
   int32_t max_iter;
+  int32_t bands;  // bands of P::rows rows a block goes through (1 where the program stores pixels)
 };
 
 struct PixIn {
@@ -83,10 +84,9 @@ __device__ constexpr bool pix_effect_op(int op) { return pix_scatter_op(op) || o
 
 // A register stored to an int32 field: truncation toward zero, NaN -> 0, saturating.
 __device__ __forceinline__ int pix_to_i32(float x) {
-  if (x != x) return 0;
-  if (x >= 2147483648.0f) return 2147483647;
-  if (x < -2147483648.0f) return -2147483647 - 1;
-  return static_cast<int>(x);
+  // selects, no branches: a branch between the rows a thread evaluates would hold their loads apart
+  const int v = static_cast<int>(fminf(fmaxf(x, -2147483648.0f), 2147483520.0f));
+  return x != x ? 0 : x >= 2147483648.0f ? 2147483647 : v;
 }
 
 // Wave sums for scatter-adds at wave-uniform indices (every lane of the wave takes part; lanes
@@ -206,6 +206,24 @@ struct PixConstAdds {
   static constexpr int N = slot(end);
 };
 
+// Adds at per-pixel indices into a block's LDS copy (P::priv) are made after all P::rows pixels of a
+// thread are evaluated, while those are few: an atomic holds back every later load, so an add per
+// row made each row wait for its own load (8192^2 f32 into 256 bins, 1024 blocks, 8 rows: 144 us, 75 here).
+template <class P>
+struct PixPending {
+  static constexpr int end = P::n_pre + P::n_test + P::n_body + P::n_post;
+  static constexpr bool may(int pc) {
+    return P::code[pc].op == VDSL_PIX_ATOMIC_ADD && !PixConstAdds<P>::at(pc) && P::priv[P::code[pc].a] > 0 &&
+           !(P::code[pc].ext[0] != 0 && P::code[pc].ext[1] != 0);
+  }
+  static constexpr int slot(int pc) {
+    int n = 0;
+    for (int q = 0; q < pc; ++q) n += may(q) ? 1 : 0;
+    return n;
+  }
+  static constexpr int N = slot(end);
+  static constexpr bool runs = P::rows > 0 && N > 0 && N * P::rows <= 32;  // two registers each
+};
 
 template <class P>
 struct PixAcc {
@@ -215,6 +233,9 @@ struct PixAcc {
   int n[N];          // adds made (none: nothing to add)
   float x[N], y[N];  // the indices (constants)
   unsigned* sh[VDSL_PIX_MAX_INPUTS];  // the block's LDS copy of input k where P::priv[k] > 0
+  static constexpr int ROWS = PixPending<P>::runs ? P::rows : 1, PN = PixPending<P>::runs ? PixPending<P>::N : 1;
+  int row;                                // of the thread's P::rows pixels, the one being evaluated
+  unsigned pe[ROWS][PN], pv[ROWS][PN];    // pending adds: element of the LDS copy (~0: none), value's bits
 };
 
 // An add into input A's element e, component c: into the block's LDS copy where A has one
@@ -233,15 +254,20 @@ __device__ __forceinline__ void pix_add(const PixIn& in, PixAcc<P>& acc, PixOff<
 // VDSL_PIX_ATOMIC_ADD into input A: component c of [x][y] += v on lanes with act set, where the
 // element is in A.  UNI: x and y are the same on every lane of the wave (host dataflow, row
 // mapping), so the wave's values are summed and one lane adds.
-template <class P, int A, bool UNI, int OP>
+template <class P, int PC, int A, bool UNI, int OP>
 __device__ __forceinline__ void pix_scatter_add(const PixIn& in, PixAcc<P>& acc, float x, float y, float v, int c, bool act) {
   bool in_a;
   const PixOff<P> e = pix_target<P, A>(in, x, y, in_a);
   const bool ok = act && in_a;
   constexpr bool i32 = P::in_dtypes[A] == VDSL_I32;
   float vf = ok && !i32 ? v : pix_none_f<OP>();
-  int vi = ok && i32 ? pix_to_i32(v) : pix_none_i<OP>();
-  if constexpr (UNI) {
+  const int wi = i32 ? pix_to_i32(v) : 0;
+  int vi = ok && i32 ? wi : pix_none_i<OP>();
+  if constexpr (PixPending<P>::runs && PixPending<P>::may(PC)) {
+    constexpr int k = PixPending<P>::slot(PC);
+    acc.pe[acc.row][k] = ok ? static_cast<unsigned>(e) * static_cast<unsigned>(P::in_widths[A]) + static_cast<unsigned>(c) : ~0u;
+    acc.pv[acc.row][k] = i32 ? static_cast<unsigned>(wi) : __float_as_uint(v);
+  } else if constexpr (UNI) {
     const uint64_t any = __builtin_amdgcn_ballot_w64(ok);
     if (any == 0ull) return;
     if constexpr (OP == VDSL_PIX_ATOMIC_ADD) {
@@ -261,19 +287,52 @@ __device__ __forceinline__ void pix_scatter_add(const PixIn& in, PixAcc<P>& acc,
   }
 }
 
+// The pending adds of a thread's P::rows pixels into the block's LDS copies.
+template <class P, int PC>
+__device__ __forceinline__ void pix_drain_one(PixAcc<P>& acc, int t) {
+  if constexpr (PixPending<P>::may(PC)) {
+    constexpr int A = P::code[PC].a, k = PixPending<P>::slot(PC);
+    if (acc.pe[t][k] == ~0u) return;
+    if constexpr (P::in_dtypes[A] == VDSL_I32) atomicAdd(reinterpret_cast<int*>(acc.sh[A]) + acc.pe[t][k], static_cast<int>(acc.pv[t][k]));
+    else atomicAdd(reinterpret_cast<float*>(acc.sh[A]) + acc.pe[t][k], __uint_as_float(acc.pv[t][k]));
+  }
+}
+
+template <class P, int... PC>
+__device__ __forceinline__ void pix_drain(PixAcc<P>& acc, Seq<PC...>) {
+  if constexpr (PixPending<P>::runs) {
+#pragma unroll
+    for (int t = 0; t < P::rows; ++t) (pix_drain_one<P, PC>(acc, t), ...);
+  }
+}
+
+// No add pending for any of a thread's pixels (those a loop leaves out stay so).
+template <class P>
+__device__ __forceinline__ void pix_none_pending(PixAcc<P>& acc) {
+  if constexpr (PixPending<P>::runs) {
+#pragma unroll
+    for (int t = 0; t < P::rows; ++t)
+#pragma unroll
+      for (int k = 0; k < PixPending<P>::N; ++k) acc.pe[t][k] = ~0u;
+  }
+}
+
 template <class P, int PC>
 __device__ __forceinline__ void pix_accumulate(PixAcc<P>& acc, float x, float y, float v, bool act) {
   constexpr vdsl_map_instr s = P::code[PC];
   constexpr int k = PixConstAdds<P>::slot(PC);
   constexpr int OP = s.op;
-  if (act) {
-    // the first value as it is (the accumulators start at 0, which is no identity of max / min)
-    if constexpr (P::in_dtypes[s.a] == VDSL_I32)
-      acc.i[k] = acc.n[k] ? pix_combine<OP>(acc.i[k], pix_to_i32(v)) : pix_to_i32(v);
-    else
-      acc.f[k] = acc.n[k] ? pix_combine<OP>(acc.f[k], v) : v;
-    acc.n[k] += 1;
+  // the first value as it is (the accumulators start at 0, which is no identity of max / min); selects,
+  // as in pix_to_i32
+  const bool first = acc.n[k] == 0;
+  if constexpr (P::in_dtypes[s.a] == VDSL_I32) {
+    const int w = pix_to_i32(v), both = pix_combine<OP>(acc.i[k], w);
+    acc.i[k] = act ? (first ? w : both) : acc.i[k];
+  } else {
+    const float both = pix_combine<OP>(acc.f[k], v);
+    acc.f[k] = act ? (first ? v : both) : acc.f[k];
   }
+  acc.n[k] += act ? 1 : 0;
   acc.x[k] = x;
   acc.y[k] = y;
 }
@@ -368,7 +427,7 @@ __device__ __forceinline__ void pix_step(const PixRt& rt, const PixIn& in, float
     // one add (max, min) per wave where both indices are the same on every lane (found
     // wave-uniform by the host in the row mapping: ext[0], ext[1]), else one per lane
     constexpr bool uni = P::rows > 0 && s.ext[0] != 0 && s.ext[1] != 0;
-    pix_scatter_add<P, s.a, uni, s.op>(in, acc, r[s.b], r[s.c], r[s.dst], static_cast<int>(rt.imm[PC]), act);
+    pix_scatter_add<P, PC, s.a, uni, s.op>(in, acc, r[s.b], r[s.c], r[s.dst], static_cast<int>(rt.imm[PC]), act);
   } else if constexpr (s.op == VDSL_MAP_LOAD) {
     r[s.dst] = pix_load<P, s.a>(in, o, s.c);
   } else if constexpr (s.op == VDSL_PIX_LOAD_AT) {
@@ -725,21 +784,28 @@ __device__ __forceinline__ void pixel_body(const PixRt& rt, const PixIn& in, voi
   if constexpr (P::rows > 0) {
     const unsigned T = xcd_band(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
     const int j = static_cast<int>((T % gridDim.x) * 256 + threadIdx.x);
-    const int i0 = static_cast<int>(T / gridDim.x) * P::rows;
+    const int i0 = static_cast<int>(T / gridDim.x) * P::rows * (P::out_kind == VDSL_PIX_OUT_NONE ? rt.bands : 1);
     if constexpr (P::out_kind == VDSL_PIX_OUT_NONE) {
       // nothing stored (a reduction into a few elements, whose blocks cover many rows so that
-      // few adds reach memory): the rows in a loop, eight at a time
-#pragma unroll 8
-      for (int t = 0; t < P::rows; ++t) {
-        if constexpr (P::loop)
-          if (i0 + t >= ni) break;
-        float unused[4];
-        int unused_count;
-        pixel_eval<P>(rt, in, ni, nj, i0 + t, j, unused, unused_count, acc);
+      // few adds reach memory): bands of P::rows rows whose loads are issued together
+      for (int i = i0; i < min(i0 + P::rows * rt.bands, ni); i += P::rows) {
+        pix_none_pending<P>(acc);
+#pragma unroll
+        for (int t = 0; t < P::rows; ++t) {
+          if constexpr (P::loop)
+            if (i + t >= ni) break;
+          acc.row = t;
+          float unused[4];
+          int unused_count;
+          pixel_eval<P>(rt, in, ni, nj, i + t, j, unused, unused_count, acc);
+        }
+        pix_drain<P>(acc, typename MakeSeq<PixPending<P>::end>::type{});
       }
     } else {
+      pix_none_pending<P>(acc);
 #pragma unroll
       for (int t = 0; t < P::rows; ++t) {
+        acc.row = t;
         // a loop is not run for the last band's rows past the grid (the same for the whole
         // block); a program without one evaluates them unconditionally, so the loads of all its
         // rows are issued together (a branch between them would order them)
@@ -747,6 +813,7 @@ __device__ __forceinline__ void pixel_body(const PixRt& rt, const PixIn& in, voi
           if (i0 + t >= ni) break;
         pixel_eval<P>(rt, in, ni, nj, i0 + t, j, res[t], count[t], acc);
       }
+      pix_drain<P>(acc, typename MakeSeq<PixPending<P>::end>::type{});
 #pragma unroll
       for (int t = 0; t < P::rows; ++t) pixel_store<P>(out, ni, nj, i0 + t, j, res[t], count[t]);
     }
