@@ -9,6 +9,7 @@ import pytest
 
 from oracle import oracle
 from vernondsl_amd import _lib, kernels, rng
+from vernondsl_amd._lib import call
 from vernondsl_amd.rhi import Tensor
 
 pytestmark = pytest.mark.gpu
@@ -48,11 +49,11 @@ def test_row_major(dev, q, M, N, K):
         t.free()
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 32, 256), (8, 96, 4096), (20, 8192, 256), (32, 544, 512), (31, 96, 512), (127, 32, 2304),
+@pytest.mark.parametrize("M,N,K", [(1, 32, 256), (8, 96, 4096), (20, 8192, 256), (32, 544, 512), (31, 96, 512), (127, 32, 2304), (16, 16384, 512), (17, 16416, 512), (24, 65536, 256),
                                    (300, 32, 2048), (2000, 32, 256)])
 def test_packed_equals_row_major(dev, q, M, N, K):
     """Packed weights, with every epilogue, against the row-major form and the separate ops, bit for
-    bit (K is split alike for all of them)."""
+    bit (every output is one chain of MFMAs over K in all of them)."""
     a, b = operands(M, N, K, M + N + K)
     ta, tb, tbp = Tensor.from_numpy(dev, q, a, "bf16"), Tensor.from_numpy(dev, q, b, "bf16"), Tensor(dev, (N, K), "bf16")
     kernels.pack_bf16_weights(q, tb, tbp)
@@ -80,6 +81,47 @@ def test_packed_equals_row_major(dev, q, M, N, K):
         assert np.array_equal(t.numpy(q), ref_t)
     for t in [ta, tb, tbp] + f + h + ht:
         t.free()
+
+
+# every configuration of the chain (1, 2 and 4 row tiles, 1 and 2 column tiles; one stage, several and a
+# part; K that ends inside a step), waves that load for themselves (K up to 128, 256 on a long side; one
+# and two row tiles; a ragged last block), both orders of the short side, and the limits of the rules:
+# 16 / 17, 32 / 33 and 127 rows, 8192 and 16384 columns
+SAME = [(1, 40, 8), (16, 512, 300), (5, 1000, 520), (17, 96, 1024), (32, 257, 2048), (16, 8200, 160), (32, 8192, 128), (17, 8193, 136),
+        (9, 65537, 256), (31, 65536, 72), (33, 96, 1040), (127, 500, 304), (64, 8192, 136), (40, 4200, 264), (300, 10, 1000),
+        (9000, 20, 64), (2000, 100, 712), (1, 1, 4096)]
+
+
+@pytest.mark.parametrize("M,N,K", SAME)
+def test_same_bits_on_every_path(dev, q, M, N, K):
+    """A short-side product equals the tile kernels' bit for bit, in all four layouts; so does each row on
+    its own (one row's result does not depend on the batch)."""
+    a, b = operands(M, N, K, M + 5 * N + K)
+
+    def product(x, y, ta, tb, config=-1):
+        m, n = len(x), len(y)
+        call("vdsl_debug_gemm_config", config)
+        try:
+            t = [Tensor.from_numpy(dev, q, np.ascontiguousarray(x.T) if ta else x, "bf16"),
+                 Tensor.from_numpy(dev, q, y if tb else np.ascontiguousarray(y.T), "bf16"), Tensor(dev, (m, n), "f32"),
+                 Tensor(dev, (max(1, kernels.gemm_bf16_workspace_bytes(ta, tb, m, n, K)),), "i8")]
+            t[2].buffer.fill_u32(q, 0x7FC00000)
+            kernels.gemm_bf16(q, t[0], t[1], t[2], ta, tb, _lib.EPI_NONE, None, t[3])
+            out = t[2].numpy(q)
+        finally:
+            call("vdsl_debug_gemm_config", -1)
+        for v in t:
+            v.free()
+        return out
+
+    got = product(a, b, False, True)
+    if K % 8 == 0:
+        assert np.array_equal(got, product(a, b, False, True, config=0))
+    for ta, tb in ((False, False), (True, False), (True, True)):
+        assert np.array_equal(got, product(a, b, ta, tb)), (ta, tb)
+    big = np.concatenate([a] * (200 // M + 1)) if M < 200 else a  # the same rows in a batch past the limit
+    assert np.array_equal(got, product(big, b, False, True)[:M])
+    assert np.array_equal(got[M // 2:M // 2 + 1], product(a[M // 2:M // 2 + 1], b, False, True))
 
 
 @pytest.mark.parametrize("M,N,K,packed", [(1, 32, 512, True), (8, 8192, 512, True), (33, 96, 4608, True), (100, 1024, 1024, True),

@@ -87,11 +87,13 @@ def test_mlp_small_end_to_end(dev, q, d_in):
         assert np.linalg.norm(a - r) <= 1e-2 * np.linalg.norm(r), n
 
 
-def test_mlp_graph_variants_identical(dev, q):
+# (batch, d_in, hidden, d_out): square tiles, a batch of short-side products, a narrow last layer
+@pytest.mark.parametrize("sizes", [(256, 512, 512, 256), (16, 512, 512, 256), (8, 256, 1024, 512), (300, 256, 256, 32)])
+def test_mlp_graph_variants_identical(dev, q, sizes):
     """The prepared-transpose, fused-GELU-backward and packed-weight forms of the training step (and
     mlp_train_graph's default, all three) run the same products in the same order: every output
     equals the plain graph's bit for bit (each graph also replays equal to its eager run)."""
-    x, w1, w2, t = spec.mlp_inputs(batch=256, d_in=512, hidden=512, d_out=256)
+    x, w1, w2, t = spec.mlp_inputs(*sizes)
     plain = {"prepare_transposes": False, "fuse_gelu_backward": False, "pack_weights": False, "fuse_mse": False,
              "store_gelu_deriv": False}
     base = run_mlp(dev, q, x, w1, w2, t, replays=2, **plain)

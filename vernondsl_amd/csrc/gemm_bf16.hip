@@ -566,37 +566,45 @@ __global__ __launch_bounds__(Cfg::THREADS) void gemm_bf16_skinny(const uint16_t*
                                                                  void* __restrict__ C, float* __restrict__ pre, int M, int N,
                                                                  int K, int kind, int epi, int c_dtype,
                                                                  uint16_t* __restrict__ ctr) {
-  __shared__ __attribute__((aligned(16))) char smem[Cfg::LDS_BYTES];
   const int cm = SWAP ? N : M, cn = SWAP ? M : N;  // C's extents
-  const unsigned tiles_n = (N + Cfg::BN - 1) / Cfg::BN;
-  skinny_gemm<Cfg>(reinterpret_cast<const char*>(A), reinterpret_cast<const char*>(B), M, N, 2 * K,
-                   static_cast<int>(blockIdx.x / tiles_n) * Cfg::BM, static_cast<int>(blockIdx.x % tiles_n) * Cfg::BN, smem, [&](int i, int j, float v) {
-                     const int row = SWAP ? j : i, col = SWAP ? i : j;
-                     if (kind == kSkinnyForward) bf16_epilogue<0>(v, row, col, cm, cn, C, pre, epi, c_dtype, ctr);
-                     else if (kind == kSkinnyGeluBwd) bf16_epilogue<1>(v, row, col, cm, cn, C, pre, epi, c_dtype, ctr);
-                     else if (kind == kSkinnyMul) bf16_epilogue<2>(v, row, col, cm, cn, C, pre, epi, c_dtype, ctr);
-                     else bf16_epilogue<0, true>(v, row, col, cm, cn, C, pre, epi, c_dtype, ctr);
-                   });
+  const unsigned tiles_n = (static_cast<unsigned>(N) + Cfg::BN - 1) / Cfg::BN;
+  const int m0 = static_cast<int>(blockIdx.x / tiles_n) * Cfg::BM, n0 = static_cast<int>(blockIdx.x % tiles_n) * Cfg::BN;
+  const char *a = reinterpret_cast<const char*>(A), *b = reinterpret_cast<const char*>(B);
+  const auto out = [&](int i, int j, float v) {
+    const int row = SWAP ? j : i, col = SWAP ? i : j;
+    if (kind == kSkinnyForward) bf16_epilogue<0>(v, row, col, cm, cn, C, pre, epi, c_dtype, ctr);
+    else if (kind == kSkinnyGeluBwd) bf16_epilogue<1>(v, row, col, cm, cn, C, pre, epi, c_dtype, ctr);
+    else if (kind == kSkinnyMul) bf16_epilogue<2>(v, row, col, cm, cn, C, pre, epi, c_dtype, ctr);
+    else bf16_epilogue<0, true>(v, row, col, cm, cn, C, pre, epi, c_dtype, ctr);
+  };
+  if constexpr (Cfg::LDS_BYTES == 0) {
+    skinny_direct<Cfg>(a, b, M, N, 2 * K, m0, n0, out);
+  } else {
+    __shared__ __attribute__((aligned(16))) char smem[Cfg::LDS_BYTES];
+    skinny_chain<Cfg>(a, b, M, N, 2 * K, m0, n0, smem, out);
+  }
 }
 
-// Whether a product takes gemm_skinny.h: a side of at most 32, or one below 128 whose long operand
-// cannot be packed, while the blocks of 64 x 32 come to at most two per CU.  The same for every operand
-// form, so all give the same bits.  us, operands rotating, packed [M][4096] x [4096][4096] with 128 x
-// 256 tiles before, here, and in 32 x 64 tiles: M = 1 42.7, 7.4; 8 43.2, 8.2; 20 44.5, 10.2, 15.4; 32
-// 45.3, 11.5, 14.2; 64 47.8, 18.5, 14.4; 127 52.6, 19.6, 16.4.  Row-major (tiles before, here): [127] 39.8,
-// 25.1; [300][1000] x [10] 17.8, 4.7.  A block reads its whole A side (43 GB/s a CU from L2), so four
-// blocks per CU lose: [127][4096] x [16384] 59 against 95.
-bool skinny_runs(int64_t M, int64_t N, int64_t K) {
+// Whether a product takes gemm_skinny.h.  Every path gives the same bits, so the rule is by time alone
+// (us, operands rotating).  Packed: up to 16 rows, up to 32 below 16384 columns: [M][4096] x [4096][4096] in
+// the tiles of bpk_dispatch and here: M = 1 18.6, 9.3; 8 19.0, 11.1; 16 19.3, 11.9; 32 18.8, 15.2; [20][4096] x
+// [16384] 28.8, 31.0; [1000][4096] x [32] 15.6, 18.1.  Row-major, in the tiles of launch_nt and here: a side
+// of at most 32 ([8][4096] x [4096] 30.2, 11.2; [300][1000] x [10] 10.8, 4.3), or below 128 while the tiles of
+// 64 x 64 leave CUs idle ([64][4000] x [4000] 30.5, 22.4; [127][300] x [500] 6.4, 4.2; [64][200] x [16000] 6.1, 8.4;
+// [127][1000] x [8000] 12.2, 15.9); of rows that are not whole 16-byte units, up to 8192 of the long side
+// ([8][1001] x [4096] 10.6, 6.8; [31][255] x [10000] 7.1, 10.6), where waves do not load for themselves.
+bool skinny_runs(bool packed, int64_t M, int64_t N, int64_t K) {
   const int64_t s = M < N ? M : N, l = M < N ? N : M;
-  const bool packable = N % 32 == 0 && K % 256 == 0;
-  return (s <= 32 || (s < 128 && !packable && ((s + 63) / 64) * ((l + 31) / 32) <= 512)) && s * K >= 8 &&
-         gemm_config_override() < 0;
+  if (s * K < 8 || l > 0x7fffff00 || gemm_config_override() >= 0) return false;
+  if (packed) return M <= 16 || (M <= 32 && (N < 16384 || direct_runs(M, N, K)));
+  if (K % 8 != 0 && l > 8192 && !direct_runs(s, l, K)) return false;
+  return s <= 32 || (s < 128 && ((s + 63) / 64) * ((l + 31) / 32) <= 256);
 }
 
 template <SkinnyForm FORM, bool SWAP>
 int launch_skinny_form(const uint16_t* A, const uint16_t* B, void* C, float* pre, int M, int N, int K, int kind, int epi, int ct,
                        hipStream_t s, uint16_t* ctr) {
-  return skinny_dispatch<Mfma16Bf16, FORM>(M, N, int64_t{2} * K, [&](auto cfg) {
+  return chain_dispatch<FORM>(M, N, K, [&](auto cfg) {
     using Cfg = decltype(cfg);
     const int64_t blocks = ((int64_t{N} + Cfg::BN - 1) / Cfg::BN) * ((int64_t{M} + Cfg::BM - 1) / Cfg::BM);
     if (blocks > 0x7fffffff) return fail(VDSL_ERR_UNSUPPORTED, "GEMM: too many tiles");
@@ -809,7 +817,7 @@ int choose_config(int64_t M, int64_t N, int64_t K) {
 
 int launch_nt(const uint16_t* A, const uint16_t* B, void* C, float* pre, int M, int N, int K, int epi, int ct, hipStream_t s,
               uint16_t* ctr = nullptr) {
-  if (skinny_runs(M, N, K))
+  if (skinny_runs(false, M, N, K))
     return launch_skinny(false, A, B, C, pre, M, N, K, epi == kEpiGeluBwd ? kSkinnyGeluBwd : kSkinnyForward, epi, ct, s, ctr);
   // Row-major operands by gemm_any.h: rows that are not whole 16-byte units (one lane per output
   // before: 300x784x1000 with K = 300, 303 us against 7), outputs of fewer than 512 tiles of 64 x 64
@@ -989,7 +997,7 @@ extern "C" int vdsl_op_gemm_bf16_packed(vdsl_queue q, int64_t M, int64_t N, int6
   VDSL_TRY(check_buffer(q, C, nbytes(M, N, dtype_size(c_dtype)), "C", true));
   if (pre_act) VDSL_TRY(check_buffer(q, pre_act, nbytes(M, N, 4), "pre_act", true));
   if (M == 0 || N == 0) return VDSL_OK;
-  if (skinny_runs(M, N, K))
+  if (skinny_runs(true, M, N, K))
     return launch_skinny(true, static_cast<const uint16_t*>(A->ptr), static_cast<const uint16_t*>(Bp->ptr), C->ptr,
                          pre_act ? static_cast<float*>(pre_act->ptr) : nullptr, static_cast<int>(M), static_cast<int>(N),
                          static_cast<int>(K), epilogue == VDSL_EPI_GELU_DERIV ? kSkinnyDeriv : kSkinnyForward, epilogue, c_dtype,
@@ -1018,7 +1026,7 @@ extern "C" int vdsl_op_gemm_bf16_gelu_bwd_packed(vdsl_queue q, int64_t M, int64_
   VDSL_TRY(check_buffer(q, da, nbytes(M, N, 2), "da", true));
   if (da_t) VDSL_TRY(check_buffer(q, da_t, nbytes(M, N, 2), "da_t", true));
   if (M == 0 || N == 0) return VDSL_OK;
-  if (skinny_runs(M, N, K))
+  if (skinny_runs(true, M, N, K))
     return launch_skinny(true, static_cast<const uint16_t*>(A->ptr), static_cast<const uint16_t*>(Bp->ptr), da->ptr,
                          static_cast<float*>(pre->ptr), static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), kSkinnyGeluBwd,
                          kEpiGeluBwd, VDSL_BF16, q->stream, da_t ? static_cast<uint16_t*>(da_t->ptr) : nullptr);
@@ -1045,7 +1053,7 @@ extern "C" int vdsl_op_gemm_bf16_mul_packed(vdsl_queue q, int64_t M, int64_t N, 
   VDSL_TRY(check_buffer(q, c, nbytes(M, N, 2), "c", true));
   if (c_t) VDSL_TRY(check_buffer(q, c_t, nbytes(M, N, 2), "c_t", true));
   if (M == 0 || N == 0) return VDSL_OK;
-  if (skinny_runs(M, N, K))
+  if (skinny_runs(true, M, N, K))
     return launch_skinny(true, static_cast<const uint16_t*>(A->ptr), static_cast<const uint16_t*>(Bp->ptr), c->ptr,
                          static_cast<float*>(g->ptr), static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), kSkinnyMul,
                          kEpiGeluBwd, VDSL_BF16, q->stream, c_t ? static_cast<uint16_t*>(c_t->ptr) : nullptr);

@@ -451,7 +451,7 @@ bool skinny_runs(int64_t M, int64_t N, int64_t K, int64_t most_rows, int64_t mos
 template <SkinnyForm FORM, bool SWAP>
 int launch_skinny(const int8_t* a, const int8_t* b, const float* xs, const float* wsc, void* y, int out_dtype, int relu,
                   int32_t* ao, int m, int n, int k, hipStream_t s) {
-  return skinny_dispatch<Mfma16I8, FORM>(m, n, k, [&](auto cfg) {
+  return skinny_dispatch<FORM>(m, n, k, [&](auto cfg) {
     using Cfg = decltype(cfg);
     const int64_t blocks = ((int64_t{n} + Cfg::BN - 1) / Cfg::BN) * ((int64_t{m} + Cfg::BM - 1) / Cfg::BM);
     if (blocks > 0x7fffffff) return fail(VDSL_ERR_UNSUPPORTED, "GEMM: too many tiles");
