@@ -126,7 +126,9 @@ def test_same_bits_on_every_path(dev, q, M, N, K):
 
 @pytest.mark.parametrize("M,N,K,packed", [(1, 32, 512, True), (8, 8192, 512, True), (33, 96, 4608, True), (100, 1024, 1024, True),
                                           (300, 64, 512, True), (1, 1, 16, False), (5, 37, 80, False), (17, 8200, 272, False),
-                                          (127, 130, 4112, False), (500, 3, 64, False), (64, 1000, 4096, False)])
+                                          (127, 130, 4112, False), (500, 3, 64, False), (64, 1000, 4096, False),
+                                          # past the rule's long sides: the tiles, and activations long
+                                          (8, 16400, 64, False), (17, 8208, 528, False), (16400, 17, 256, False)])
 def test_int8(dev, q, M, N, K, packed):
     r = np.random.default_rng(M * 5 + N + K)
     xq = r.integers(-127, 128, (M, K)).astype(np.int8)

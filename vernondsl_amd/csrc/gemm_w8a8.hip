@@ -11,9 +11,10 @@
 // the accumulator layout is the f32 one.  This file adds the dequant epilogue and the split-K path.
 //
 // Products with a short side (a few rows of activations) run gemm_skinny.h.  Other narrow outputs
-// (too few tiles to fill 256 CUs, e.g. the 1024-wide last layer at batch 512) split K across blocks: each block adds its int32 partial tile into a zeroed int32 workspace
-// with atomics - integer addition is exact and order-independent, so the result is still
-// deterministic - and a second kernel applies the dequant epilogue.
+// (too few tiles to fill 256 CUs, e.g. the 1024-wide last layer at batch 512) split K across blocks:
+// each block adds its int32 partial tile into a zeroed int32 workspace with atomics - integer addition
+// is exact and order-independent, so the result is still deterministic - and a second kernel applies
+// the dequant epilogue.
 
 #include "gemm_bpk.h"
 #include "gemm_dma.h"
@@ -426,7 +427,7 @@ __global__ __launch_bounds__(Cfg::THREADS) void gemm_w8a8_skinny(const int8_t* _
                                                                  void* __restrict__ y, int out_dtype, int relu,
                                                                  int32_t* __restrict__ acc_out, int M, int N, int K) {
   __shared__ __attribute__((aligned(16))) char smem[Cfg::LDS_BYTES];
-  const unsigned tiles_n = (N + Cfg::BN - 1) / Cfg::BN;
+  const unsigned tiles_n = (static_cast<unsigned>(N) + Cfg::BN - 1) / Cfg::BN;
   skinny_gemm<Cfg>(reinterpret_cast<const char*>(A), reinterpret_cast<const char*>(B), M, N, K,
                    static_cast<int>(blockIdx.x / tiles_n) * Cfg::BM, static_cast<int>(blockIdx.x % tiles_n) * Cfg::BN, smem, [&](int i, int j, int32_t a) {
                      const int row = SWAP ? j : i, col = SWAP ? i : j;
@@ -436,16 +437,29 @@ __global__ __launch_bounds__(Cfg::THREADS) void gemm_w8a8_skinny(const int8_t* _
                    });
 }
 
-// Whether a product takes gemm_skinny.h: a short side of at most `most_rows`, or below 128 with K up
-// to `most_k` (a block reads its whole A side, the split-K tiles a part of it), and at most two blocks
-// of 64 x 32 per CU.  Packed, us, weights rotating, tiles before: [8][8192] x [8192] 24.5 -> 13.1, [32]
-// 24.7 -> 15.4, [8][8192] x [1024] 12.6 -> 6.7, [127][2048] x [2048] 9.5 -> 7.4; but [64][8192] x [1024]
-// 12.9 -> 18.4, [127][8192] x [8192] 28.9 -> 40.0: 32 rows or K of 2048.  Row-major: [64][2000] x [2000]
-// 10.7 -> 6.6, [8][8192] x [8192] 18.2 -> 16.3, [100][4096] x [4096] 14.4 either way: 64 rows or 4096.
-bool skinny_runs(int64_t M, int64_t N, int64_t K, int64_t most_rows, int64_t most_k) {
+// Whether a product takes gemm_skinny.h: a short side of at most 32, or below 128 with K up to `most_k` (a
+// block reads its whole A side, the split-K tiles a part of it), and at most two blocks of 64 x 32 per CU.
+// Packed, K of 2048, us, weights rotating, tiles before: [8][8192] x [8192] 24.5 -> 13.1, [32] 24.7 -> 15.4,
+// [8][8192] x [1024] 12.6 -> 6.7, [127][2048] x [2048] 9.5 -> 7.4; but [64][8192] x [1024] 12.9 -> 18.4,
+// [127][8192] x [8192] 28.9 -> 40.0.
+bool skinny_fits(int64_t M, int64_t N, int64_t K, int64_t most_k) {
   const int64_t s = M < N ? M : N, l = M < N ? N : M;
-  return s < 128 && (s <= most_rows || K <= most_k) && (s <= 32 || ((s + 63) / 64) * ((l + 31) / 32) <= 512) && K >= 16 &&
+  return s < 128 && (s <= 32 || (K <= most_k && ((s + 63) / 64) * ((l + 31) / 32) <= 512)) && K >= 16 && l <= 0x7fffff00 &&
          gemm_config_override() < 0;
+}
+
+// Row-major operands, which the tiles read as well as this kernel does once they cover the CUs.  Up to
+// 8192 of the long side (4096 above 64 rows: [100][1024] x [8192] 13.7 -> 15.1), K of 4096 for up to 64 rows of
+// activations ([64][4096] x [8192] 18.9 -> 16.5, but [4096][4096] x [64] 11.9 -> 12.8, [100][4096] x [4096] 14.0 ->
+// 14.4): [64][2000] x [2000] 10.7 -> 6.6, [8][8192] x [8192] 18.2 -> 16.3.  Beyond, while the weights are the
+// long side and no longer than 16384 ([8][64] x [1000000] 61 -> 106, [8][1024] x [30000] 10.6 -> 14.6), up to 16
+// rows or K of 512 ([16][2048] x [16384] 15.0 -> 9.6, [32][512] x [16384] 10.4 -> 7.2; but [32][1024] x [10000] 9.9
+// -> 10.6), and where the activations are, up to 16 columns or 32 with K of 256 ([1000000][64] x [8] 128 -> 106,
+// [1000000][128] x [31] 230 -> 201; but [60000][512] x [31] 22.1 -> 24.2, [10000][512] x [64] 8.8 -> 12.2).
+bool skinny_rows_run(int64_t M, int64_t N, int64_t K) {
+  const int64_t s = M < N ? M : N, l = M < N ? N : M;
+  if (!skinny_fits(M, N, K, M <= N && s <= 64 ? 4096 : 2048) || (s > 64 && l > 4096)) return false;
+  return l <= 8192 || (M > N ? s <= 16 || (s <= 32 && K <= 256) : l <= 16384 && (s <= 16 || K <= 512));
 }
 
 template <SkinnyForm FORM, bool SWAP>
@@ -792,7 +806,7 @@ extern "C" int vdsl_op_gemm_w8a8(vdsl_queue q, int64_t M, int64_t N, int64_t K, 
   const auto* b = static_cast<const int8_t*>(w->ptr);
   const auto* xs = static_cast<const float*>(x_scale->ptr);
   const auto* wsc = static_cast<const float*>(w_scale->ptr);
-  if (skinny_runs(M, N, K, 64, 4096)) {
+  if (skinny_rows_run(M, N, K)) {
     if (m <= n) return launch_skinny<kSkinnyRows, false>(a, b, xs, wsc, y->ptr, out_dtype, relu, ao, m, n, k, q->stream);
     return launch_skinny<kSkinnyRows, true>(b, a, xs, wsc, y->ptr, out_dtype, relu, ao, n, m, k, q->stream);
   }
@@ -866,7 +880,7 @@ static int packed_launch(vdsl_queue q, const BpkPlan& p, int64_t M, int64_t N, i
   const auto* xs = static_cast<const float*>(x_scale->ptr);
   const auto* wsc = static_cast<const float*>(w_scale->ptr);
   const int m = static_cast<int>(M), n = static_cast<int>(N), k = static_cast<int>(K);
-  if (skinny_runs(M, N, K, 32, 2048) && g_bpk_plan.load(std::memory_order_relaxed) < 0)
+  if (skinny_fits(M, N, K, 2048) && g_bpk_plan.load(std::memory_order_relaxed) < 0)
     return launch_skinny<kSkinnyPacked, false>(a, b, xs, wsc, y->ptr, out_dtype, relu, ao, m, n, k, q->stream);
   if (p.cfg == 0) return launch_bpk<P0>(p, a, b, xs, wsc, y->ptr, out_dtype, relu, ao, part, m, n, k, q->stream);
   if (p.cfg == 3) return launch_bpk<P3>(p, a, b, xs, wsc, y->ptr, out_dtype, relu, ao, part, m, n, k, q->stream);
