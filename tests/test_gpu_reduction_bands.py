@@ -44,3 +44,38 @@ def test_bands(dev, q, ni, nj, n, dtype, store):
         assert np.array_equal(out.numpy(q), x)
     for t in [tx, total] + ts + ([out] if store else []):
         t.free()
+
+
+def int_program(bins, n, total, per_row):
+    """target k < n: [0][floor(x * bins) + k] += k + 1, or with per_row [0][floor(i / 128)] += 1; with total,
+    an int32 sum of 16 x at a constant index."""
+    b = pp.Builder()
+    x = b.load(0)
+    at = b.op("floor", b.op("mul", b.index(0), 1.0 / 128)) if per_row else b.op("floor", b.op("mul", x, float(bins)))
+    fx = [b.scatter_add(1 + k, 0.0, b.op("add", at, float(k)) if k else at, float(k + 1)) for k in range(n)]
+    if total:
+        fx.append(b.scatter_add(1 + n, 0.0, 0.0, b.op("mul", x, 16.0)))
+    return pp.compile_program(b, effects=fx, in_dtypes=[pp.F32] + [pp.I32] * (n + total),
+                              in_extents=[None] + [(1, bins)] * n + [(1, 1)] * total)
+
+
+# grids of more bands of 8 rows than a launch's y extent (65535), up to the most rows a program may have;
+# f32 totals (64 rows a block) and int32 ones
+@pytest.mark.parametrize("ni, nj", [(524281, 1), (600000, 3), (1048560, 1)])
+@pytest.mark.parametrize("f32", [True, False])
+def test_tall(dev, q, ni, nj, f32):
+    bins, n = 100, 3
+    r = np.random.default_rng(ni)
+    x = (r.integers(-2, 18, (ni, nj)) / 16.0 * (r.random((ni, nj)) < 0.25)).astype(np.float32)
+    at = np.floor(x.astype(np.float64) * bins).astype(int)
+    tx, total = Tensor.from_numpy(dev, q, x), Tensor.from_numpy(dev, q, np.zeros((1, 1), np.float32 if f32 else np.int32))
+    ts = [Tensor.from_numpy(dev, q, np.full((1, bins), k, np.int32)) for k in range(n)]
+    prog = program(bins, n, pp.I32, False) if f32 else int_program(bins, n, 1, False)
+    kernels.pixel_program(q, prog, [tx] + ts + [total], None, grid=(ni, nj))
+    for k, t in enumerate(ts):
+        e = (at + k)[(at + k >= 0) & (at + k < bins)]
+        assert np.array_equal(t.numpy(q).astype(np.int64)[0], k + (k + 1) * np.bincount(e, minlength=bins))
+    assert np.abs(x).sum(dtype=np.float64) < 2 ** 20
+    assert total.numpy(q)[0, 0] == x.sum(dtype=np.float64) * (1 if f32 else 16)
+    for t in [tx, total] + ts:
+        t.free()

@@ -164,14 +164,16 @@ int rows_per_block(const vdsl_pixel_program& p, const std::vector<char>& flags, 
   return gathers ? 8 : 4;
 }
 
-// Blocks of rows x 256 pixels for programs whose pixels all do the same work (no
-// escape loop), while the row count fits the grid's y extent; 16x16 patches otherwise.  0 for
-// the patches.
+// Blocks of rows x 256 pixels for programs whose pixels all do the same work (no escape loop), while
+// the row count fits the grid's y extent; 16x16 patches otherwise.  0 for the patches.  A reduction's
+// blocks go through as many bands of `rows` rows as that extent takes (make_plan).
+constexpr int kMaxGridY = 65535;
 int row_mapping(const vdsl_pixel_program& p, const std::vector<char>& flags, bool reduction, int ni) {
   // never more rows per block than the grid has: a 1-D field is a grid of one row, whose blocks
   // would otherwise run their loops for rows that do not exist
   const int rows = std::min(rows_per_block(p, flags, reduction), std::max(ni, 1));
-  return !(p.loop && p.test != VDSL_PIX_TEST_NONE) && (ni + rows - 1) / rows <= 65535 ? rows : 0;
+  if (p.loop && p.test != VDSL_PIX_TEST_NONE) return 0;
+  return reduction || (ni + rows - 1) / rows <= kMaxGridY ? rows : 0;
 }
 
 // Bands of `rows` rows per block of a reduction.  Adds of many blocks to one element are serialised
@@ -308,7 +310,12 @@ Plan make_plan(const vdsl_pixel_program& p, int n_inputs, int ni, int nj) {
   }
   const bool reduction = is_reduction(p, pl.flags, pl.priv);
   pl.rows = row_mapping(p, pl.flags, reduction, ni);
-  if (reduction && pl.rows) pl.bands = std::min(reduction_bands(p, pl.flags, pl.rows, ni, nj), (ni + pl.rows - 1) / pl.rows);
+  if (reduction && pl.rows) {
+    // tall grids: bands of 8 rows, one a block, over 600000 rows do not fit the grid, and in patches each
+    // 16 x 16 pixels add to memory on their own (600000x64, three histograms: 2800 us, 203 in 64 rows a block)
+    const int all = (ni + pl.rows - 1) / pl.rows;
+    pl.bands = std::max(std::min(reduction_bands(p, pl.flags, pl.rows, ni, nj), all), (all + kMaxGridY - 1) / kMaxGridY);
+  }
   return pl;
 }
 
