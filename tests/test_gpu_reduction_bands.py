@@ -59,6 +59,27 @@ def int_program(bins, n, total, per_row):
                               in_extents=[None] + [(1, bins)] * n + [(1, 1)] * total)
 
 
+# int32 targets alone: the root rule gives 2 to 3 bands a block on the first four grids (the last block's of
+# fewer rows, or of fewer bands), adds at row-uniform indices several once 4096 units of a band are passed
+@pytest.mark.parametrize("ni, nj, n, total, per_row", [(1500, 1027, 1, 0, False), (1505, 1027, 2, 1, False), (1501, 1027, 3, 1, False),
+                                                       (4099, 700, 0, 1, False), (8203, 2050, 1, 0, True), (8203, 2050, 1, 1, True)])
+def test_int32_bands(dev, q, ni, nj, n, total, per_row):
+    bins = 100
+    x = (np.random.default_rng(ni + n).integers(-2, 18, (ni, nj)) / 16.0).astype(np.float32)
+    tx = Tensor.from_numpy(dev, q, x)
+    ts = [Tensor.from_numpy(dev, q, np.full((1, bins), k, np.int32)) for k in range(n)]
+    sums = [Tensor.from_numpy(dev, q, np.zeros((1, 1), np.int32))] if total else []
+    kernels.pixel_program(q, int_program(bins, n, total, per_row), [tx] + ts + sums, None, grid=(ni, nj))
+    at = np.repeat(np.arange(ni) // 128, nj) if per_row else np.floor(x.astype(np.float64) * bins).astype(int)
+    for k, t in enumerate(ts):
+        e = (at + k)[(at + k >= 0) & (at + k < bins)]
+        assert np.array_equal(t.numpy(q).astype(np.int64)[0], k + (k + 1) * np.bincount(e, minlength=bins))
+    for t in sums:
+        assert t.numpy(q)[0, 0] == int((x.astype(np.float64) * 16).sum())
+    for t in [tx] + ts + sums:
+        t.free()
+
+
 # grids of more bands of 8 rows than a launch's y extent (65535), up to the most rows a program may have;
 # f32 totals (64 rows a block) and int32 ones
 @pytest.mark.parametrize("ni, nj", [(524281, 1), (600000, 3), (1048560, 1)])

@@ -178,15 +178,20 @@ int row_mapping(const vdsl_pixel_program& p, const std::vector<char>& flags, boo
 
 // Bands of `rows` rows per block of a reduction.  Adds of many blocks to one element are serialised
 // (~13 ns each) while few blocks leave CUs and loads in flight short, so the best count grows as the
-// root of the pixels.  us with blocks of 64 rows (their adds one by one), and 256, 512, 768, 1024, 2048
-// blocks: 1885x5071, 256 bins 35.2; 25.6, 21.6, 22.8, 24.1, 29.9; 2603x6098, 369 bins 42.7; 38.6, 27.7,
-// 28.4, 30.9, 46.5; 8192x8192, 256 bins 129.0; 139, 81.8, 69.1, 63.8, 73.8.  Small grids had few
+// root of the pixels (over 8, or 256).  us with blocks of 64 rows (their adds one by one), and 256, 512,
+// 768, 1024, 2048 blocks: 1885x5071, 256 bins 35.2; 25.6, 21.6, 22.8, 24.1, 29.9; 2603x6098, 369 bins 42.7; 38.6,
+// 27.7, 28.4, 30.9, 46.5; 8192x8192, 256 bins 129.0; 139, 81.8, 69.1, 63.8, 73.8.  Small grids had few
 // blocks: 777x1460, 1009 bins 16.2, here 11.2 (its two launches take about 10 from the host).
+// Programs of three adds or more, whose bands are of 8 rows, do best with twice the blocks (8192x8192 130 us
+// with the root's 1024, 116; 1885x5071 38.1, 36.6), on one column of blocks, where a block is a chain of
+// LDS adds by few waves, with no more than 64 rows in each (600000x64 245, 222).  Columns count in whole blocks of
+// 256 (600000x3, 100 bins: 340 us counting its pixels, 148 counting its lanes, 199 with blocks of 64 rows).
 // f32 sums keep 64 rows a block, and with them the lengths of the chains they are added in, and so do
 // programs with more adds than PixPending holds.  Where int32 adds are wave-uniform (made row by row, as
 // many whatever the block's rows), the block's waves wait on each: one band while that gives at most 4096
-// blocks, else at least 1024 blocks.  Row sums, blocks of 64 rows and here: 1024x1024 29.1, 9.6 us; 2000x5000
-// 42.1, 24.5 (420 blocks 62.7); 8192x8192 219, 209 (one band, whose LDS copies cost more: 259).
+// blocks, else 64 rows.  Sums over ranges of rows, blocks of 64 rows with their adds one by one, and here:
+// 1000x3 33.1, 9.3 us; 1885x5071 50.1, 37.6; 600000x3 198, 161 (1024 blocks 284); 8192x8192 132, 99.6 (1024 blocks
+// 127), two of them 188, 167 (216).
 int reduction_bands(const vdsl_pixel_program& p, const std::vector<char>& flags, int rows, int ni, int nj) {
   if (const int r = rows_override()) return (r + rows - 1) / rows;
   const int total = p.n_pre + p.n_test + p.n_body + p.n_post;
@@ -200,9 +205,11 @@ int reduction_bands(const vdsl_pixel_program& p, const std::vector<char>& flags,
   }
   if (sums || pending * rows > 32) return (std::min(64, ni) + rows - 1) / rows;
   const int64_t units = ((nj + 255) / 256) * static_cast<int64_t>((ni + rows - 1) / rows);
-  if (uniform) return units <= 4096 ? 1 : static_cast<int>(std::min<int64_t>(units / 1024, ni));
-  const double blocks = std::max(256.0, std::sqrt(static_cast<double>(ni) * nj) / 8);
-  return static_cast<int>(std::min(std::max(1.0, units / blocks + 0.5), static_cast<double>(ni)));
+  if (uniform) return units <= 4096 ? 1 : (64 + rows - 1) / rows;
+  const double lanes = 256.0 * rows * static_cast<double>(units);
+  const double blocks = std::max(256.0, (pending > 2 ? 2 : 1) * std::sqrt(lanes) / 8);
+  const double most = pending > 2 && nj <= 256 ? (64 + rows - 1) / rows : ni;
+  return static_cast<int>(std::min(std::max(1.0, units / blocks + 0.5), most));
 }
 
 // Registers an instruction reads (a, b, c as the opcode uses them).
