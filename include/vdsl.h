@@ -134,11 +134,16 @@ int vdsl_buffer_copy(vdsl_queue q, vdsl_buffer dst, size_t dst_offset, vdsl_buff
                      size_t src_offset, size_t bytes);
 
 /* ---- queues ------------------------------------------------------------------------------ */
+/* A queue holds 1 MiB of device memory for partial results of vdsl_op_col_reduce, which takes no
+ * workspace (a queue that cannot have it runs that op without, more slowly). */
 int vdsl_queue_create(vdsl_device dev, vdsl_queue* out);
 int vdsl_queue_destroy(vdsl_queue q);
 int vdsl_queue_sync(vdsl_queue q);
 
 /* ---- execution-graph replay (one hipGraph per recorded op sequence) ------------------------ */
+/* Allocates the same 1 MiB for the recording, before it begins (kept by the queue from one recording
+ * to the next until a recorded op uses it; the graph then owns it and frees it when destroyed).
+ * Neither the recorded op calls nor the replays allocate. */
 int vdsl_graph_begin(vdsl_queue q);
 int vdsl_graph_end(vdsl_queue q, vdsl_graph* out);
 int vdsl_graph_launch(vdsl_graph g, vdsl_queue q);
@@ -464,7 +469,9 @@ int vdsl_op_mat_transform(vdsl_queue q, int64_t n, int32_t dim, int32_t in_width
 int vdsl_op_row_reduce_softmax(vdsl_queue q, int64_t rows, int64_t cols, int32_t dtype,
                                vdsl_buffer x, vdsl_buffer row_sum, vdsl_buffer row_max,
                                vdsl_buffer softmax);
-/* Column reductions of an f32/bf16 [rows][cols] tensor: col_sum, col_max f32 [cols] (either NULL). */
+/* Column reductions of an f32/bf16 [rows][cols] tensor: col_sum, col_max f32 [cols] (either NULL).
+ * Large tensors are reduced in ranges of rows whose f64 sums meet in scratch memory (vdsl_queue_create);
+ * without it in one range: the f64 sums are then grouped otherwise. */
 int vdsl_op_col_reduce(vdsl_queue q, int64_t rows, int64_t cols, int32_t dtype, vdsl_buffer x,
                        vdsl_buffer col_sum, vdsl_buffer col_max);
 
@@ -617,7 +624,8 @@ int vdsl_op_gemm_w8a8_packed_noalloc(vdsl_queue q, int64_t M, int64_t N, int64_t
 
 /* ---- failure injection (tests of error paths, host-side only) ----------------------------- */
 /* After `n` more successful buffer allocations, the next one fails with VDSL_ERR_OUT_OF_MEMORY
- * (n < 0 disables).  Also settable with the environment variable VDSL_FAIL_ALLOC_AFTER. */
+ * (n < 0 disables).  While n is 0, queues and recordings get no scratch memory either (which fails
+ * no call).  Also settable with the environment variable VDSL_FAIL_ALLOC_AFTER. */
 int vdsl_debug_fail_alloc_after(int64_t n);
 
 /* ---- tuning hook (tests and sweeps, host-side only) ----------------------------------------- */

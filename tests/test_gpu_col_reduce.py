@@ -8,6 +8,7 @@ import pytest
 
 from oracle import oracle
 from vernondsl_amd import kernels, rng
+from vernondsl_amd._lib import call
 from vernondsl_amd.rhi import Queue, Tensor
 
 pytestmark = pytest.mark.gpu
@@ -92,4 +93,61 @@ def test_recorded_and_on_two_queues(dev, q):
     rec.graph.destroy()
     other.destroy()
     for t in tx + [t for o in out for t in o]:
+        t.free()
+
+
+def test_while_another_queue_records(dev):
+    """A queue made, its first reduction, and a graph with scratch freed while another queue of the thread
+    records: all succeed, the recording too, with the results of the same calls alone."""
+    x = rng.normal(3, 9000 * 512).reshape(9000, 512)
+    a = Queue(dev)
+    tx = Tensor.from_numpy(dev, a, x)
+    out = [(Tensor(dev, (512,), "f32"), Tensor(dev, (512,), "f32")) for _ in range(2)]
+    kernels.col_reduce(a, tx, *out[0])
+    ref = out[0][0].numpy(a), out[0][1].numpy(a)
+    with a.capture() as old:
+        kernels.col_reduce(a, tx, *out[1])
+    with a.capture() as rec:
+        b = Queue(dev)
+        kernels.col_reduce(b, tx, *out[1])
+        kernels.col_reduce(a, tx, *out[0])
+        old.graph.destroy()
+    assert np.array_equal(out[1][0].numpy(b), ref[0]) and np.array_equal(out[1][1].numpy(b), ref[1])
+    for _ in range(3):
+        for t in out[0]:
+            t.buffer.fill_u32(a, 0x7FC00000)
+        rec.graph.launch(a)
+        assert np.array_equal(out[0][0].numpy(a), ref[0]) and np.array_equal(out[0][1].numpy(a), ref[1])
+    rec.graph.destroy()
+    b.destroy()
+    a.destroy()
+    for t in [tx] + [t for o in out for t in o]:
+        t.free()
+
+
+@pytest.mark.parametrize("shape", [(9000, 512), (20000, 77)])
+def test_without_scratch(dev, q, shape):
+    """A queue and a recording that get no scratch memory: one range of rows, right all the same."""
+    x = rng.normal(5, shape[0] * shape[1]).reshape(shape)
+    out = [Tensor(dev, (shape[1],), "f32") for _ in range(4)]
+    tx = Tensor.from_numpy(dev, q, x)
+    call("vdsl_debug_fail_alloc_after", 0)
+    try:
+        a = Queue(dev)
+        with a.capture() as rec:
+            kernels.col_reduce(a, tx, *out[2:])
+    finally:
+        call("vdsl_debug_fail_alloc_after", -1)
+    kernels.col_reduce(a, tx, *out[:2])
+    for _ in range(2):
+        for t in out[2:]:
+            t.buffer.fill_u32(a, 0x7FC00000)
+        rec.graph.launch(a)
+        a.sync()
+    check(x, out[0].numpy(a), out[1].numpy(a))
+    for t, u in zip(out[:2], out[2:]):
+        assert np.array_equal(t.numpy(a), u.numpy(a))
+    rec.graph.destroy()
+    a.destroy()
+    for t in [tx] + out:
         t.free()

@@ -6,7 +6,6 @@
 
 #include <atomic>
 #include <string>
-#include <vector>
 
 #include "fmath.h"
 #include "vdsl.h"
@@ -40,8 +39,10 @@ struct vdsl_queue_s {
   vdsl_device dev;
   hipStream_t stream;
   bool capturing;
-  void* scratch = nullptr;            // queue_scratch(): kept from the first op that asks for it
-  std::vector<void*> graph_scratch;   // asked for by the ops recorded since vdsl_graph_begin
+  void* scratch = nullptr;        // queue_scratch() of the ops that run on it
+  void* graph_scratch = nullptr;  // of the ops recorded since vdsl_graph_begin, which allocates it; kept
+                                  // for the next recording where no op asked for it
+  bool graph_scratch_used = false;
 };
 
 struct vdsl_graph_s {
@@ -49,7 +50,7 @@ struct vdsl_graph_s {
   vdsl_device dev;
   hipGraph_t graph;
   hipGraphExec_t exec;
-  std::vector<void*> scratch;  // of its ops; freed with it
+  void* scratch = nullptr;  // of its ops, if one asked for it; freed with it
 };
 
 struct vdsl_event_s {
@@ -79,13 +80,13 @@ int check_buffer(vdsl_queue q, vdsl_buffer b, size_t bytes, const char* name, bo
 
 size_t dtype_size(int dtype);
 
-// Device memory for one op's partial results on queue q, valid until the queue's next op: the
-// queue's own kQueueScratchBytes, allocated when first asked for, or, while q records a graph, a
-// piece of its own that the graph then owns (so graphs replayed on any queues share nothing).
-// *out is null, with VDSL_OK, when `bytes` is more than that or cannot be had: the op then takes
-// the path that needs none.
+// Device memory for one op's partial results on queue q, kQueueScratchBytes valid until the queue's next
+// op: the queue's own, allocated by vdsl_queue_create, or, while q records a graph, that of the graph,
+// allocated by vdsl_graph_begin and the graph's from vdsl_graph_end on (its ops run in order; graphs
+// replayed on any queues share nothing).  So no op allocates, in a recording or out of one.  Null when
+// `bytes` is more than that or could not be had: the op then takes the path that needs none.
 constexpr size_t kQueueScratchBytes = size_t{1} << 20;
-int queue_scratch(vdsl_queue q, size_t bytes, void** out);
+void* queue_scratch(vdsl_queue q, size_t bytes);
 
 // Per-device set-up of the allocation-free int8 GEMM (gemm_w8a8.hip); called by vdsl_device_open
 // with the device current.

@@ -651,9 +651,7 @@ int launch_cols(vdsl_queue q, const void* x, float* cs, float* cm, int64_t rows,
     if (want > 1) {
       per_range = (rows + want - 1) / want;
       ranges = static_cast<int>((rows + per_range - 1) / per_range);
-      void* scratch = nullptr;
-      VDSL_TRY(queue_scratch(q, nbytes(ranges, cols, 12), &scratch));
-      part = static_cast<double*>(scratch);
+      part = static_cast<double*>(queue_scratch(q, nbytes(ranges, cols, 12)));
     }
   }
   if (!part) {

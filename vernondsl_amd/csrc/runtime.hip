@@ -109,30 +109,38 @@ int check_buffer(vdsl_queue q, vdsl_buffer b, size_t bytes, const char* name, bo
   return VDSL_OK;
 }
 
-int queue_scratch(vdsl_queue q, size_t bytes, void** out) {
-  *out = nullptr;
-  if (!bytes || bytes > kQueueScratchBytes) return VDSL_OK;
-  if (!q->capturing) {
-    if (!q->scratch && hipMalloc(&q->scratch, kQueueScratchBytes) != hipSuccess) {
-      (void)hipGetLastError();
-      q->scratch = nullptr;
-    }
-    *out = q->scratch;
-    return VDSL_OK;
-  }
-  // An allocation does not touch the recording; the thread's capture mode has to allow it.
+namespace {
+
+// The library's own device memory, allocated and freed while another queue may be recording on this
+// thread: HIP refuses both then, unless the thread's capture mode is relaxed (neither touches a
+// recording).  Null where it cannot be had.
+void* scratch_alloc() {
+  if (fail_alloc_budget() == 0) return nullptr;
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-  VDSL_TRY(check_hip(hipThreadExchangeStreamCaptureMode(&mode), "hipThreadExchangeStreamCaptureMode"));
+  if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return nullptr;
   void* p = nullptr;
-  const hipError_t e = hipMalloc(&p, bytes);
-  VDSL_TRY(check_hip(hipThreadExchangeStreamCaptureMode(&mode), "hipThreadExchangeStreamCaptureMode"));
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
-    return VDSL_OK;
-  }
-  q->graph_scratch.push_back(p);
-  *out = p;
-  return VDSL_OK;
+  if (hipMalloc(&p, kQueueScratchBytes) != hipSuccess) p = nullptr;
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  (void)hipGetLastError();
+  return p;
+}
+
+void scratch_free(void* p) {
+  if (!p) return;
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  (void)hipFree(p);
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  (void)hipGetLastError();
+}
+
+}  // namespace
+
+void* queue_scratch(vdsl_queue q, size_t bytes) {
+  if (!bytes || bytes > kQueueScratchBytes) return nullptr;
+  if (!q->capturing) return q->scratch;
+  q->graph_scratch_used = q->graph_scratch != nullptr;
+  return q->graph_scratch;
 }
 
 size_t dtype_size(int dtype) {
@@ -362,6 +370,7 @@ int vdsl_queue_create(vdsl_device dev, vdsl_queue* out) {
   q->dev = dev;
   q->stream = s;
   q->capturing = false;
+  q->scratch = scratch_alloc();
   dev->live.fetch_add(1);
   reg_add(q);
   *out = q;
@@ -374,7 +383,8 @@ int vdsl_queue_destroy(vdsl_queue q) {
   (void)hipSetDevice(q->dev->ordinal);
   int st = check_hip(hipStreamSynchronize(q->stream), "hipStreamSynchronize");
   (void)hipStreamDestroy(q->stream);
-  if (q->scratch) (void)hipFree(q->scratch);
+  scratch_free(q->scratch);
+  scratch_free(q->graph_scratch);
   reg_del(q);
   q->dev->live.fetch_sub(1);
   q->magic = 0;
@@ -393,6 +403,8 @@ int vdsl_queue_sync(vdsl_queue q) {
 int vdsl_graph_begin(vdsl_queue q) {
   VDSL_TRY(enter_queue(q));
   if (q->capturing) return fail(VDSL_ERR_CAPTURE, "queue is already capturing");
+  if (!q->graph_scratch) q->graph_scratch = scratch_alloc();
+  q->graph_scratch_used = false;
   VDSL_TRY(check_hip(hipStreamBeginCapture(q->stream, hipStreamCaptureModeThreadLocal),
                      "hipStreamBeginCapture"));
   q->capturing = true;
@@ -404,27 +416,16 @@ int vdsl_graph_end(vdsl_queue q, vdsl_graph* out) {
   VDSL_TRY(enter_queue(q));
   if (!q->capturing) return fail(VDSL_ERR_CAPTURE, "graph_end without graph_begin");
   q->capturing = false;
-  std::vector<void*> scratch;
-  scratch.swap(q->graph_scratch);
-  auto drop = [&]() {
-    for (void* p : scratch) (void)hipFree(p);
-  };
   hipGraph_t g = nullptr;
-  int st = check_hip(hipStreamEndCapture(q->stream, &g), "hipStreamEndCapture");
-  if (st != VDSL_OK) {
-    drop();
-    return st;
-  }
+  VDSL_TRY(check_hip(hipStreamEndCapture(q->stream, &g), "hipStreamEndCapture"));
   if (!out) {
     (void)hipGraphDestroy(g);
-    drop();
     return fail(VDSL_ERR_INVALID_ARG, "out is null (recording discarded)");
   }
   hipGraphExec_t exec = nullptr;
-  st = check_hip(hipGraphInstantiate(&exec, g, nullptr, nullptr, 0), "hipGraphInstantiate");
+  int st = check_hip(hipGraphInstantiate(&exec, g, nullptr, nullptr, 0), "hipGraphInstantiate");
   if (st != VDSL_OK) {
     (void)hipGraphDestroy(g);
-    drop();
     return st;
   }
   auto* gr = new vdsl_graph_s();
@@ -432,7 +433,10 @@ int vdsl_graph_end(vdsl_queue q, vdsl_graph* out) {
   gr->dev = q->dev;
   gr->graph = g;
   gr->exec = exec;
-  gr->scratch = std::move(scratch);
+  if (q->graph_scratch_used) {
+    gr->scratch = q->graph_scratch;
+    q->graph_scratch = nullptr;
+  }
   q->dev->live.fetch_add(1);
   reg_add(gr);
   *out = gr;
@@ -452,7 +456,7 @@ int vdsl_graph_destroy(vdsl_graph g) {
   (void)hipSetDevice(g->dev->ordinal);
   (void)hipGraphExecDestroy(g->exec);
   (void)hipGraphDestroy(g->graph);
-  for (void* p : g->scratch) (void)hipFree(p);
+  scratch_free(g->scratch);
   reg_del(g);
   g->dev->live.fetch_sub(1);
   g->magic = 0;
