@@ -16,7 +16,9 @@ pytestmark = pytest.mark.gpu
 # one row; fewer rows than row lanes; a partial batch; a last row range of one row (4097 over 256-row
 # ranges); strips past the last column; odd, even and 16-byte widths; enough bytes for several ranges
 SHAPES = [(1, 1), (1, 5), (3, 64), (63, 260), (1000, 333), (4097, 256), (4097, 72), (16384, 3), (8193, 130), (2049, 1031),
-          (300, 16384), (5, 40000)]
+          (300, 16384), (5, 40000), (64, 32768), (8, 1 << 20), (33, 65544),
+          # few rows: a lane per column or vector, small and wide, ragged; the widest strips of 1024 lanes
+          (12, 333), (16, 70001), (17, 70001), (7, 600008), (2, 1100002), (9, 300000), (65, 131080)]
 
 
 def check(xf, cs, cm):

@@ -490,15 +490,15 @@ struct ColLoad {
   }
 };
 
-template <int DT, int VEC>
-__global__ __launch_bounds__(kColThreads) void col_reduce_kernel(const void* __restrict__ x, float* __restrict__ col_sum,
+template <int DT, int VEC, int THREADS>
+__global__ __launch_bounds__(THREADS) void col_reduce_kernel(const void* __restrict__ x, float* __restrict__ col_sum,
                                                                  float* __restrict__ col_max, double* __restrict__ part_sum,
                                                                  float* __restrict__ part_max, int64_t all_rows, int64_t per_range,
                                                                  int64_t cols, int lg_lanes) {
   using LD = ColLoad<DT, VEC>;
   using Raw = typename LD::Raw;
-  extern __shared__ __align__(16) char col_smem[];  // [16][L * VEC] f64 sums, then as many f32 maxima
-  const int L = 1 << lg_lanes, width = VEC << lg_lanes, R = kColThreads >> lg_lanes;
+  extern __shared__ __align__(16) char col_smem[];  // [waves][L * VEC] f64 sums, then as many f32 maxima
+  const int L = 1 << lg_lanes, width = VEC << lg_lanes, R = THREADS >> lg_lanes;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int64_t strip = blockIdx.x, first = static_cast<int64_t>(blockIdx.y) * per_range;
   const int64_t rows = all_rows - first < per_range ? all_rows - first : per_range;  // of this range
@@ -557,7 +557,7 @@ __global__ __launch_bounds__(kColThreads) void col_reduce_kernel(const void* __r
     }
   }
   double* const ssum = reinterpret_cast<double*>(col_smem);
-  float* const smax = reinterpret_cast<float*>(ssum + (kColThreads / 64) * width);
+  float* const smax = reinterpret_cast<float*>(ssum + (THREADS / 64) * width);
   if (lane < L) {
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
@@ -566,13 +566,13 @@ __global__ __launch_bounds__(kColThreads) void col_reduce_kernel(const void* __r
     }
   }
   __syncthreads();
-  for (int k = threadIdx.x; k < width; k += kColThreads) {
+  for (int k = threadIdx.x; k < width; k += THREADS) {
     const int64_t col = strip * width + k;
     if (col >= cols) break;
     double t = ssum[k];
     float mm = smax[k];
 #pragma unroll
-    for (int w = 1; w < kColThreads / 64; ++w) {
+    for (int w = 1; w < THREADS / 64; ++w) {
       t += ssum[w * width + k];
       mm = fmaxf(mm, smax[w * width + k]);
     }
@@ -583,6 +583,55 @@ __global__ __launch_bounds__(kColThreads) void col_reduce_kernel(const void* __r
       if (col_sum) col_sum[col] = static_cast<float>(t);
       if (col_max) col_max[col] = mm;
     }
+  }
+}
+
+// Few rows: a lane per VEC columns takes all of them, 8 rows' loads at a time; nothing to combine.  Up to 8
+// rows, or 16 of small tensors; us with the lanes of a block split over rows (most of them idle, then LDS
+// and butterflies) and here: [1][1000000] f32 47.6, 4.7 bf16 27.4, 3.7; [2][3000001] f32 143, 9.9; [8][1048576]
+// bf16 24.1, 6.7; [16][30000] f32 5.0, 2.6; but [16][2000000] bf16 18.0 in blocks of 256 lanes split over rows, 21.7.
+template <int DT, int VEC>
+__global__ __launch_bounds__(256) void col_few_kernel(const void* __restrict__ x, float* __restrict__ col_sum,
+                                                      float* __restrict__ col_max, int rows, int64_t pitch) {
+  using LD = ColLoad<DT, VEC>;
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;  // of the row's loads
+  if (i >= pitch) return;
+  const typename LD::Raw* src = reinterpret_cast<const typename LD::Raw*>(x) + i;
+  double s[VEC];
+  float m[VEC];
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) s[e] = 0.0, m[e] = -INFINITY;
+  for (int r = 0; r < rows; r += kColBatch) {
+    std::conditional_t<LD::kBytes == 2, uint32_t, typename LD::Raw> v[kColBatch];  // (no halves of one register)
+#pragma unroll
+    for (int u = 0; u < kColBatch; ++u)
+      if (r + u < rows) v[u] = src[(r + u) * pitch];
+#pragma unroll
+    for (int u = 0; u < kColBatch; ++u) {
+      if (r + u >= rows) break;
+      float f[VEC];
+      LD::unpack(static_cast<typename LD::Raw>(v[u]), f);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) {
+        s[e] += static_cast<double>(f[e]);
+        m[e] = fmaxf(m[e], f[e]);
+      }
+    }
+  }
+  struct __attribute__((packed, aligned(4))) Out {
+    float v[VEC];
+  };
+  if (col_sum) {
+    Out o;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) o.v[e] = static_cast<float>(s[e]);
+    reinterpret_cast<Out*>(col_sum)[i] = o;
+  }
+  if (col_max) {
+    Out o;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) o.v[e] = m[e];
+    reinterpret_cast<Out*>(col_max)[i] = o;
   }
 }
 
@@ -628,10 +677,11 @@ __global__ __launch_bounds__(kColThreads) void col_finish_kernel(const double* _
 // with 256 blocks (512: 30.0); [16384][256] f32 8.5 us against 31 us in one launch.  For less the
 // second launch costs more than the strips' latency ([700][700] f32 6.8 us a call against 5.4; but
 // [16384][64] 7.2 against 21.7, hence the row count): one range, and strips narrowed to 16 bytes
-// while they do not cover the CUs and a row lane has more than half a
-// batch of rows.  Those read an element or a bf16 pair per lane (col_small): with 16 bytes per lane
-// the f64 adds and butterflies of few blocks take longer than the loads ([100][16384] bf16 5.1 us a
-// call against 4.1).
+// while they do not cover the CUs and a row lane has more than half a batch of rows.  Up to 64 rows
+// such a block has 256 lanes (of 1024 most have no row: [20][262144] f32 10.5 us against 6.2,
+// [64][1048576] bf16 46.2 against 32.2).  Small tensors are read an element or a bf16 pair per lane
+// (col_small): with 16 bytes per lane the f64 adds and butterflies of few blocks take longer than the
+// loads ([100][16384] bf16 5.1 us a call against 4.1).
 bool col_small(int64_t rows, int64_t bytes) {
   return !(bytes >= (int64_t{4} << 20) || (bytes >= (int64_t{1} << 20) && rows >= 4096));
 }
@@ -641,6 +691,13 @@ int launch_cols(vdsl_queue q, const void* x, float* cs, float* cm, int64_t rows,
   constexpr int kBytes = ColLoad<DT, VEC>::kBytes;
   const auto strips = [&](int l) { return (cols + (int64_t{VEC} << l) - 1) / (int64_t{VEC} << l); };
   const int64_t bytes = rows * cols * (DT == VDSL_F32 ? 4 : 2);  // fits: checked by the caller
+  if (rows <= (col_small(rows, bytes) ? 16 : 8)) {
+    const int64_t pitch = cols / VEC, threads = pitch < 256 * 256 ? 64 : 256, blocks = (pitch + threads - 1) / threads;
+    if (blocks > 0x7fffffff) return fail(VDSL_ERR_UNSUPPORTED, "too many columns");
+    hipLaunchKernelGGL((col_few_kernel<DT, VEC>), dim3(static_cast<unsigned>(blocks)), dim3(static_cast<unsigned>(threads)), 0,
+                       q->stream, x, cs, cm, static_cast<int>(rows), pitch);
+    return check_launch("col_few_kernel");
+  }
   int lg = kBytes == 16 ? 4 : 6, ranges = 1;
   int64_t per_range = rows;
   double* part = nullptr;
@@ -654,16 +711,19 @@ int launch_cols(vdsl_queue q, const void* x, float* cs, float* cm, int64_t rows,
       part = static_cast<double*>(queue_scratch(q, nbytes(ranges, cols, 12)));
     }
   }
+  const bool few = !part && rows <= 64;
+  const int threads = few ? 256 : kColThreads;
   if (!part) {
     ranges = 1, per_range = rows, lg = 6;
-    while (lg > 0 && (kBytes << (lg - 1)) >= 16 && strips(lg) < 256 && rows > (kColBatch / 2) * (kColThreads >> lg)) --lg;
+    while (lg > 0 && (kBytes << (lg - 1)) >= 16 && strips(lg) < 256 && rows > (kColBatch / 2) * (threads >> lg)) --lg;
   }
   const int64_t blocks = strips(lg);
   if (blocks > 0x7fffffff) return fail(VDSL_ERR_UNSUPPORTED, "too many columns");
   float* pmax = part ? reinterpret_cast<float*>(part + static_cast<int64_t>(ranges) * cols) : nullptr;
-  const unsigned lds = static_cast<unsigned>((kColThreads / 64) * (VEC << lg) * 12);
-  hipLaunchKernelGGL((col_reduce_kernel<DT, VEC>), dim3(static_cast<unsigned>(blocks), static_cast<unsigned>(ranges)),
-                     dim3(kColThreads), lds, q->stream, x, cs, cm, part, pmax, rows, per_range, cols, lg);
+  const unsigned lds = static_cast<unsigned>((threads / 64) * (VEC << lg) * 12);
+  hipLaunchKernelGGL((few ? col_reduce_kernel<DT, VEC, 256> : col_reduce_kernel<DT, VEC, kColThreads>),
+                     dim3(static_cast<unsigned>(blocks), static_cast<unsigned>(ranges)), dim3(threads), lds, q->stream, x, cs, cm, part,
+                     pmax, rows, per_range, cols, lg);
   VDSL_TRY(check_launch("col_reduce_kernel"));
   if (!part) return VDSL_OK;
   hipLaunchKernelGGL(col_finish_kernel, dim3(static_cast<unsigned>((cols + 63) / 64)), dim3(kColThreads), 0, q->stream, part, pmax,
