@@ -924,8 +924,11 @@ extern "C" int vdsl_op_gemm_bf16(vdsl_queue q, int32_t trans_a, int32_t trans_b,
   // Transposed operands read as stored (gemm_any.h) instead of transposing them into the workspace
   // first (1000x784x300 TN 24.8 us against 7.2, 2048^3 40.2 against 31.1, 2000x4096x4096 94.2 against 92.7),
   // but for outputs large enough that the direct-to-LDS tiles repay the transposes (4032x4096x2048 TN
-  // 87.0 against 97.6, 8000x8192x4096 522 against 657).
-  const bool large = K % 32 == 0 && ((M + 127) / 128) * ((N + 127) / 128) > 768;
+  // 87.0 against 97.6, 8000x8192x4096 522 against 657; 3056x4080x1024, 768 tiles, NN 51.6 against 55.1, TN
+  // 53.9, 56.1) and, where B alone is transposed, those whose 128 x 128 tiles are a few more than the CUs (NN
+  // 3952x1136x4096, 279 tiles, 69.7 against 77.7; 2032x2160x1024, 272, 27.8, 30.0; 2544x2032x1024, 320, 30.8, 30.5).
+  const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128);
+  const bool large = K % 32 == 0 && (t128 >= 768 || (!ta && t128 > 256 && t128 <= 304));
   if (any_runs(M, N, K) && (ta || !tb) && !large)
     return launch_any(ta, tb, a, b, C->ptr, pre, static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), epi, c_dtype,
                       q->stream);
