@@ -40,9 +40,9 @@ def _front(t, rows, cols):
 
 
 @pytest.mark.parametrize("bf16", [False, True])
-@pytest.mark.parametrize("cols", WIDTHS)
-def test_widths(dev, q, cols, bf16):
-    rows = 7 if cols > 300 else 261
+# 17 to 256 columns run the streaming kernel up to 2000 rows
+@pytest.mark.parametrize("cols, rows", [(c, 7 if c > 300 else 261) for c in WIDTHS] + [(c, 2001) for c in WIDTHS if 16 < c <= 300])
+def test_widths(dev, q, cols, rows, bf16):
     x = rng.normal(cols, rows * cols, 0.0, 2.0).reshape(rows, cols)
     x[rows // 2, cols // 2] += np.float32(20.0)
     x[0, 0] -= np.float32(100.0)  # a subnormal share where the row has other elements
@@ -63,7 +63,7 @@ def test_widths(dev, q, cols, bf16):
         assert np.all(np.abs(gsm.astype(np.float64) - p) <= (1e-6 + 2.0 ** -24 * np.abs(n)) * p + 1e-44)
 
 
-@pytest.mark.parametrize("cols", [5, 70, 1001, 5003])
+@pytest.mark.parametrize("cols", [5, 70, 300, 1001, 5003])
 def test_special_values(dev, q, cols):
     """Rows with NaN, +inf or only -inf are NaN throughout, as x - max gives; -inf elements are 0; the
     neighbouring rows, whose ends share a vector with them, are not touched."""
