@@ -161,7 +161,7 @@ def test_transpose_and_cast(dev, q):
 
 # (70, 33): the element-wise kernel; the others the 16-byte kernel (rows % 8 == 0, cols % 4 == 0),
 # (72, 100) and (8, 4) with partial tiles
-@pytest.mark.parametrize("rows,cols", [(128, 192), (70, 33), (72, 100), (8, 4), (2048, 4096)])
+@pytest.mark.parametrize("rows,cols", [(128, 192), (70, 33), (72, 100), (8, 4), (2048, 4096), (2049, 2050)])
 def test_gelu_bwd(dev, q, rows, cols):
     dh = rng.normal(21, rows * cols).reshape(rows, cols) * np.float32(1e-3)
     pre = rng.normal(22, rows * cols, 0, 2).reshape(rows, cols)
@@ -235,7 +235,7 @@ def test_add_rejects_mismatches(dev, q):
         t.free()
 
 
-@pytest.mark.parametrize("rows,cols", [(128, 192), (70, 33), (72, 100), (8, 4), (2048, 4096)])
+@pytest.mark.parametrize("rows,cols", [(128, 192), (70, 33), (72, 100), (8, 4), (2048, 4096), (2049, 2050)])
 def test_mse(dev, q, rows, cols):
     y = rng.normal(31, rows * cols).reshape(rows, cols)
     t = rng.normal(32, rows * cols).reshape(rows, cols)

@@ -169,13 +169,16 @@ __global__ __launch_bounds__(256) void mse_tile_vec(const float* __restrict__ y,
   store_pair_tile_transposed(tile, dy_t, rows, cols, r0, c0);
 }
 
-// A lane's 16 elements of two tensors, rows r, r + 4, ... of column c, all loaded before any is used
+// N of a lane's elements of two tensors, rows r, r + 4, ... of column c, all loaded before any is used
 // (rows and columns past the end repeat the last one; a branch around each load waits for it: the MSE
-// of [300][10] 7.1 us with it, 3.8 without).
+// of [300][10] 7.1 us with it, 6.0 without).  All 16 at once cost large tensors waves: us with branches,
+// 16 and 8, GELU's backward of [4001][4001] 47.4, 50.2, 48.2, of [300][10] 8.0, 5.9, 5.8; the MSE of [4001][4001]
+// 50.8, 52.4, 50.4, of [300][10] 7.0, 6.0, 6.4 (16 up to 1024 tiles).
+template <int N>
 __device__ __forceinline__ void load_column(const float* __restrict__ p, const float* __restrict__ q, int64_t r, int64_t c,
-                                            int64_t rows, int64_t cols, float (&a)[16], float (&b)[16]) {
+                                            int64_t rows, int64_t cols, float (&a)[N], float (&b)[N]) {
 #pragma unroll
-  for (int k = 0; k < 16; ++k) {
+  for (int k = 0; k < N; ++k) {
     const int64_t o = (r + 4 * k < rows ? r + 4 * k : rows - 1) * cols + (c < cols ? c : cols - 1);
     a[k] = p[o];
     b[k] = q[o];
@@ -190,15 +193,20 @@ __global__ __launch_bounds__(256) void act_bwd_kernel(const float* __restrict__ 
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
   const int64_t r0 = static_cast<int64_t>(blockIdx.y) * 64, c0 = static_cast<int64_t>(blockIdx.x) * 64;
   const int64_t c = c0 + tx;
-  float g[16], x[16];
-  load_column(dh, pre, r0 + ty, c, rows, cols, g, x);
+  constexpr int N = 8;
+#pragma unroll 1
+  for (int p0 = 0; p0 < 16; p0 += N) {
+    float g[N], x[N];
+    load_column(dh, pre, r0 + ty + 4 * p0, c, rows, cols, g, x);
 #pragma unroll
-  for (int p = 0; p < 16; ++p) {
-    const int64_t r = r0 + ty + 4 * p;
-    if (r < rows && c < cols) {
-      const uint16_t h = f32_to_bf16(act_bwd<ACT>(g[p], x[p]));
-      da[r * cols + c] = h;
-      tile[ty + 4 * p][tx] = h;
+    for (int k = 0; k < N; ++k) {
+      const int p = p0 + k;
+      const int64_t r = r0 + ty + 4 * p;
+      if (r < rows && c < cols) {
+        const uint16_t h = f32_to_bf16(act_bwd<ACT>(g[k], x[k]));
+        da[r * cols + c] = h;
+        tile[ty + 4 * p][tx] = h;
+      }
     }
   }
   if (!da_t) return;  // uniform across the block
@@ -210,6 +218,7 @@ __global__ __launch_bounds__(256) void act_bwd_kernel(const float* __restrict__ 
   }
 }
 
+template <int N>
 __global__ __launch_bounds__(256) void mse_tile_kernel(const float* __restrict__ y, const float* __restrict__ t,
                                                        uint16_t* __restrict__ dy, uint16_t* __restrict__ dy_t,
                                                        double* __restrict__ partials, int64_t rows, int64_t cols,
@@ -220,17 +229,21 @@ __global__ __launch_bounds__(256) void mse_tile_kernel(const float* __restrict__
   const int64_t r0 = static_cast<int64_t>(blockIdx.y) * 64, c0 = static_cast<int64_t>(blockIdx.x) * 64;
   double s = 0.0;
   const int64_t c = c0 + tx;
-  float a[16], b[16];
-  load_column(y, t, r0 + ty, c, rows, cols, a, b);
+#pragma unroll 1
+  for (int p0 = 0; p0 < 16; p0 += N) {
+    float a[N], b[N];
+    load_column(y, t, r0 + ty + 4 * p0, c, rows, cols, a, b);
 #pragma unroll
-  for (int p = 0; p < 16; ++p) {
-    const int64_t r = r0 + ty + 4 * p;
-    if (r < rows && c < cols) {
-      const float d = a[p] - b[p];
-      s += static_cast<double>(d) * static_cast<double>(d);
-      const uint16_t h = f32_to_bf16(d * scale);
-      if (dy) dy[r * cols + c] = h;
-      tile[ty + 4 * p][tx] = h;
+    for (int k = 0; k < N; ++k) {
+      const int p = p0 + k;
+      const int64_t r = r0 + ty + 4 * p;
+      if (r < rows && c < cols) {
+        const float d = a[k] - b[k];
+        s += static_cast<double>(d) * static_cast<double>(d);
+        const uint16_t h = f32_to_bf16(d * scale);
+        if (dy) dy[r * cols + c] = h;
+        tile[ty + 4 * p][tx] = h;
+      }
     }
   }
 #pragma unroll
@@ -374,7 +387,7 @@ extern "C" int vdsl_op_mse_fwd_bwd(vdsl_queue q, int64_t rows, int64_t cols, vds
                        static_cast<const float*>(t->ptr), dy ? static_cast<uint16_t*>(dy->ptr) : nullptr,
                        dy_t ? static_cast<uint16_t*>(dy_t->ptr) : nullptr, part, rows, cols, scale);
   else
-    hipLaunchKernelGGL(mse_tile_kernel, grid, dim3(256), 0, q->stream,
+    hipLaunchKernelGGL((np <= 1024 ? mse_tile_kernel<16> : mse_tile_kernel<8>), grid, dim3(256), 0, q->stream,
                        static_cast<const float*>(y->ptr), static_cast<const float*>(t->ptr),
                        dy ? static_cast<uint16_t*>(dy->ptr) : nullptr, dy_t ? static_cast<uint16_t*>(dy_t->ptr) : nullptr, part,
                        rows, cols, scale);
