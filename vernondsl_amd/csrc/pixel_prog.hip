@@ -305,6 +305,7 @@ struct Plan {
   int32_t priv[VDSL_PIX_MAX_INPUTS] = {}, priv_off[VDSL_PIX_MAX_INPUTS] = {};
   int32_t priv_total = 0;
   int rows = 0, bands = 1;
+  bool banded = false;  // a reduction: its blocks go through `bands` bands
 };
 
 Plan make_plan(const vdsl_pixel_program& p, int n_inputs, int ni, int nj) {
@@ -317,7 +318,8 @@ Plan make_plan(const vdsl_pixel_program& p, int n_inputs, int ni, int nj) {
   }
   const bool reduction = is_reduction(p, pl.flags, pl.priv);
   pl.rows = row_mapping(p, pl.flags, reduction, ni);
-  if (reduction && pl.rows) {
+  pl.banded = reduction && pl.rows;
+  if (pl.banded) {
     // tall grids: bands of 8 rows, one a block, over 600000 rows do not fit the grid, and in patches each
     // 16 x 16 pixels add to memory on their own (600000x64, three histograms: 2800 us, 203 in 64 rows a block)
     const int all = (ni + pl.rows - 1) / pl.rows;
@@ -342,6 +344,7 @@ std::string program_source(const vdsl_pixel_program& p, const Plan& pl, int n_in
   c("out_kind", p.out_kind);
   c("out_width", p.out_width);
   c("rows", pl.rows);
+  c("banded", pl.banded);
   // 32-bit element offsets when every field's byte offsets stay below 2^32
   int maxw = p.out_width;
   for (int k = 0; k < n_inputs; ++k) maxw = p.in_widths[k] > maxw ? p.in_widths[k] : maxw;

@@ -784,11 +784,13 @@ __device__ __forceinline__ void pixel_body(const PixRt& rt, const PixIn& in, voi
   if constexpr (P::rows > 0) {
     const unsigned T = xcd_band(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
     const int j = static_cast<int>((T % gridDim.x) * 256 + threadIdx.x);
-    const int i0 = static_cast<int>(T / gridDim.x) * P::rows * (P::out_kind == VDSL_PIX_OUT_NONE ? rt.bands : 1);
+    const int bands = P::banded ? rt.bands : 1;
+    const int i0 = static_cast<int>(T / gridDim.x) * P::rows * bands;
     if constexpr (P::out_kind == VDSL_PIX_OUT_NONE) {
       // nothing stored (a reduction into a few elements, whose blocks cover many rows so that
       // few adds reach memory): bands of P::rows rows whose loads are issued together
-      for (int i = i0; i < min(i0 + P::rows * rt.bands, ni); i += P::rows) {
+      const int end = P::banded ? min(i0 + P::rows * bands, ni) : i0 + P::rows;
+      for (int i = i0; i < end; i += P::rows) {
         pix_none_pending<P>(acc);
 #pragma unroll
         for (int t = 0; t < P::rows; ++t) {
