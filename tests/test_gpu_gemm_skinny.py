@@ -49,7 +49,7 @@ def test_row_major(dev, q, M, N, K):
         t.free()
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 32, 256), (8, 96, 4096), (20, 8192, 256), (32, 544, 512), (31, 96, 512), (127, 32, 2304), (16, 16384, 512), (17, 16416, 512), (24, 65536, 256),
+@pytest.mark.parametrize("M,N,K", [(1, 32, 256), (8, 96, 4096), (20, 8192, 256), (32, 544, 512), (31, 96, 512), (127, 32, 2304), (16, 16384, 512), (17, 16416, 512), (24, 65536, 256), (9, 65536, 256),
                                    (300, 32, 2048), (2000, 32, 256)])
 def test_packed_equals_row_major(dev, q, M, N, K):
     """Packed weights, with every epilogue, against the row-major form and the separate ops, bit for
@@ -89,7 +89,7 @@ def test_packed_equals_row_major(dev, q, M, N, K):
 # 16 / 17, 32 / 33 and 127 rows, 8192 and 16384 columns
 SAME = [(1, 40, 8), (16, 512, 300), (5, 1000, 520), (17, 96, 1024), (32, 257, 2048), (16, 8200, 160), (32, 8192, 128), (17, 8193, 136),
         (9, 65537, 256), (31, 65536, 72), (33, 96, 1040), (127, 500, 304), (64, 8192, 136), (40, 4200, 264), (300, 10, 1000),
-        (9000, 20, 64), (2000, 100, 712), (1, 1, 4096)]
+        (9000, 20, 64), (5000, 7, 40), (2000, 100, 712), (1, 1, 4096)]
 
 
 @pytest.mark.parametrize("M,N,K", SAME)

@@ -639,7 +639,10 @@ using Pb4 = BpkConfig<MfmaBf16, 1, 1, 2, 3>;  // 32 x 64 blocks, 2 waves of 32 x
 // the 256 CUs times the tile's rows and columns; a smaller tile is taken where that is less by a tenth
 // or more.  K = 4096, N = 4096, us for 128 x 256 and the choice: M = 64 47.8, 14.4 (32 x 64); 128 40.6, 15.2
 // (32 x 64); 300 46.5, 26.3 (64 x 128); 512 51.5, 28.7 (64 x 128); 2048 65.9 (128 x 256; 128 x 128 78.7);
-// [2048][4096] x [1024] 41.7, 22.7 (64 x 128), [512][2048] x [2048] 23.5, 10.9 (64 x 64).
+// [2048][4096] x [1024] 41.7, 22.7 (64 x 128), [512][2048] x [2048] 23.5, 10.9 (64 x 64).  The backward forms gain
+// alike, though tiles below 64 columns a wave store their outputs element by element: GELU backward with the
+// transposed output, [64][4096] x [4096] 87, 21.7; [300] 123, 34; [2048][4096] x [1024] 69, 36.7; times a factor 81,
+// 20.3; 112, 32.9; 60, 35.7.
 template <class Go>
 int bpk_dispatch(int64_t M, int64_t N, Go&& go) {
   const auto tiles = [&](int bm, int bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
